@@ -8,6 +8,7 @@
 // and its L2 holds the rows the stencil revisits.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <array>
 #include <cmath>
 #include <cstdarg>
@@ -22,6 +23,7 @@
 #include "qcell.h"
 #include "qsweep.h"
 #include "ql_launch.h"
+#include "psplit_launch.h"
 #include "qline_moments.h"
 #include "adjoint.h"
 #include "adjoint_lines.h"
@@ -512,6 +514,56 @@ static bool qc_applies(const boltx_grid* g) {
 
 static size_t qc_workspace_bytes(int nslab) { return 2 * (size_t)nslab * 64 * sizeof(int); }
 
+// ---- p-advection in two kernels (psplit.h) -----------------------------------
+// D, what the first kernel leaves for the second, covers a chunk of q2 rows of
+// at most this many bytes (at least one row): one chunk but for the largest
+// problems, whose workspace it bounds.  Smaller chunks, whose D and u would
+// stay in the 256 MB last-level cache, lose more in the kernels' last waves:
+// 64^2 x 24^3 in FP64 took 4.58 ms per step in chunks of 64 MB, 4.24 at 128,
+// 3.80 at 256 and 3.67 in one.
+constexpr size_t kSplitChunk = (size_t)2048 << 20;
+// The same for the library's scratch array, whose 64 MiB hold the rest too.
+constexpr size_t kSplitChunkScratch = (size_t)40 << 20;
+
+// Cells from which the two-kernel stage is the faster one.
+constexpr double kSplitCells = 786432;
+
+// Workspace of the reference layout: the sign-grouped p order, then (with the
+// two-kernel stage) D and the partial currents.
+struct RefWorkspace {
+  int rows = 0;  // q2 rows per chunk; 0: the two-kernel stage does not apply
+  size_t o_D = 0, o_part = 0, total = 0;
+};
+
+static size_t align256(size_t x) { return (x + 255) / 256 * 256; }
+
+// The two-kernel stage takes p-advection with a (p1, p2) plane of one
+// workgroup's threads, a row of D that the scratch array holds (both entry
+// points then agree bit for bit), and enough cells that the kernels' time, not
+// the second launch, is what counts.  Whole steps, one kernel / two: 256 K cells
+// 192 / 207 us in FP64 and 172 / 192 in FP32, 460 K 210 / 222 and 222 / 201,
+// 1.2 M 309 / 249 and 513 / 207, 3.5 M 590 / 356 and 313 / 260.
+static RefWorkspace ref_workspace(const boltx_grid* g, const boltx_physics* ph, size_t chunk) {
+  RefWorkspace w;
+  if (!qc_applies(g)) return w;
+  w.total = qc_workspace_bytes(qc_nslab(g));
+  if (!ph->p_advection || g->n_p1 < 2 || g->n_p2 < 2 || g->n_p3 < 2 ||
+      (long)g->n_p1 * g->n_p2 > 1024 || g->n_q1 < 2 ||
+      (double)g->n_p1 * g->n_p2 * g->n_p3 * g->n_q1 * g->n_q2 < kSplitCells)
+    return w;
+  const size_t P = (size_t)g->n_p1 * g->n_p2 * g->n_p3;
+  const size_t row = P * g->n_q1 * (ph->precision == BOLTX_FP64 ? 8 : 4);
+  const size_t prow = (P + 63) / 64 * 3 * sizeof(double) * g->n_q1;
+  if (row + prow > kSplitChunkScratch) return w;
+  const long most = std::max(1L, (long)(chunk / (row + prow)));
+  const long nchunk = (g->n_q2 + most - 1) / most;
+  w.rows = (int)((g->n_q2 + nchunk - 1) / nchunk);
+  w.o_D = align256(w.total);
+  w.o_part = align256(w.o_D + row * w.rows);
+  w.total = align256(w.o_part + prow * w.rows);
+  return w;
+}
+
 // LDS bytes of qsweep_kernel: tables, the padded p-block and its accumulator.
 static size_t qsweep_lds(const StageParams& sp) {
   const size_t pp = (size_t)(sp.n_p1 + 1) * sp.n_p2 * sp.n_p3;
@@ -754,7 +806,7 @@ static int currents_of(const StageParams& sp, const boltx_physics* phys, double*
 
 // One stage with the given workspace (the caller's, or the scratch array).
 static int fvm_stage_impl(const boltx_grid* grid, const boltx_physics* phys,
-                          const boltx_stage* st, void* workspace, hipStream_t s) {
+                          const boltx_stage* st, void* workspace, size_t chunk, hipStream_t s) {
   StageParams sp = base_params(grid);
   sp.riemann_q = phys->riemann_q;
   sp.riemann_p = phys->riemann_p;
@@ -784,6 +836,18 @@ static int fvm_stage_impl(const boltx_grid* grid, const boltx_physics* phys,
     if (phys->precision == BOLTX_FP64) return ql_stage<double>(grid, phys, st, workspace, sp, s);
     return ql_stage<float>(grid, phys, st, workspace, sp, s);
   }
+  // (currents of a grid with ghost rows: the slab kernel)
+  if (const RefWorkspace w = ref_workspace(grid, phys, chunk);
+      workspace && w.rows > 0 && !(st->currents_out && ghost_rows(grid) > 0)) {
+    char* ws = (char*)workspace;
+    void* D = ws + w.o_D;
+    double* part = (double*)(ws + w.o_part);
+    if (phys->precision == BOLTX_FP64)
+      return psplit_stage<double>(sp, phys->recon_q, phys->recon_p, w.rows, D, part,
+                                  st->currents_out, s);
+    return psplit_stage<float>(sp, phys->recon_q, phys->recon_p, w.rows, D, part,
+                               st->currents_out, s);
+  }
   if (workspace && qc_applies(grid)) {
     // the slab kernels accumulate the currents of u with the moments
     QCParams qp;
@@ -806,7 +870,7 @@ extern "C" int boltx_fvm_stage(const boltx_grid* grid, const boltx_physics* phys
                                const boltx_stage* st, void* stream) {
   int rc = check_stage(grid, phys, st);
   if (rc) return rc;
-  return fvm_stage_impl(grid, phys, st, st->workspace, (hipStream_t)stream);
+  return fvm_stage_impl(grid, phys, st, st->workspace, kSplitChunk, (hipStream_t)stream);
 }
 
 static Coeff coeff_of(const boltx_coeff& c) {
@@ -949,8 +1013,7 @@ extern "C" int boltx_fill_ghosts(const boltx_grid* grid, const boltx_physics* ph
 extern "C" size_t boltx_workspace_size(const boltx_grid* grid, const boltx_physics* phys) {
   if (check_grid(grid) || check_physics(phys)) return 0;
   if (grid->layout == BOLTX_LAYOUT_Q1_LINES) return ql_workspace_bytes(grid, phys->precision);
-  if (!qc_applies(grid)) return 0;
-  return qc_workspace_bytes(qc_nslab(grid));
+  return ref_workspace(grid, phys, kSplitChunk).total;
 }
 
 // The sign-grouped p order of the reference layout, written into the first
@@ -1012,7 +1075,9 @@ extern "C" int boltx_fvm_stage_noalloc(const boltx_grid* grid, const boltx_physi
   if (rc) return rc;
   if (st->workspace)
     return fail(BOLTX_EINVAL, "workspace must be NULL: this entry uses the library's scratch");
-  const size_t need = boltx_workspace_size(grid, phys);
+  const size_t need = grid->layout == BOLTX_LAYOUT_Q1_LINES
+                          ? ql_workspace_bytes(grid, phys->precision)
+                          : ref_workspace(grid, phys, kSplitChunkScratch).total;
   if (need > (size_t)BOLTX_SCRATCH_BYTES)
     return fail(BOLTX_EUNSUPPORTED,
                 "the problem needs %zu bytes of workspace, above the %zu of the scratch array",
@@ -1024,7 +1089,7 @@ extern "C" int boltx_fvm_stage_noalloc(const boltx_grid* grid, const boltx_physi
     // the previous call may have left another problem's p order here
     if (grid->layout == BOLTX_LAYOUT_REFERENCE && (rc = init_slab_perm(grid, ws, s))) return rc;
   }
-  return fvm_stage_impl(grid, phys, st, ws, s);
+  return fvm_stage_impl(grid, phys, st, ws, kSplitChunkScratch, s);
 }
 
 template <typename T>
@@ -1053,6 +1118,27 @@ extern "C" int boltx_currents(const boltx_grid* grid, const boltx_physics* phys,
   hipStream_t s = (hipStream_t)stream;
   if (phys->precision == BOLTX_FP64) return launch_currents<double>(sp, phys->recon_q, J, s);
   return launch_currents<float>(sp, phys->recon_q, J, s);
+}
+
+extern "C" int boltx_currents_ws(const boltx_grid* grid, const boltx_physics* phys, const void* u,
+                                 double* J, void* workspace, void* stream) {
+  int rc = check_grid(grid);
+  if (rc) return rc;
+  if ((rc = check_physics(phys))) return rc;
+  if (!u || !J) return fail(BOLTX_EINVAL, "currents pointers missing");
+  if (grid->layout != BOLTX_LAYOUT_REFERENCE)
+    return fail(BOLTX_EUNSUPPORTED, "currents need the reference layout");
+  const RefWorkspace w = ref_workspace(grid, phys, kSplitChunk);
+  if (!workspace || w.rows == 0 || ghost_rows(grid) > 0)
+    return boltx_currents(grid, phys, u, J, stream);
+  StageParams sp = base_params(grid);
+  sp.u = u;
+  sp.charge = phys->charge;
+  double* part = (double*)((char*)workspace + w.o_part);
+  hipStream_t s = (hipStream_t)stream;
+  if (phys->precision == BOLTX_FP64)
+    return psplit_currents<double>(sp, phys->recon_q, w.rows, part, J, s);
+  return psplit_currents<float>(sp, phys->recon_q, w.rows, part, J, s);
 }
 
 extern "C" int boltx_fdtd_step(const boltx_grid* grid, double* yee, const double* J, double dt,

@@ -1,0 +1,8 @@
+// FP64 instances of the two-kernel stage with p-advection.
+#define BX_PSPLIT_INSTANTIATE
+#include "psplit_launch.h"
+
+namespace bx {
+template int psplit_stage<double>(const StageParams&, int, int, int, void*, double*, double*, hipStream_t);
+template int psplit_currents<double>(const StageParams&, int, int, double*, double*, hipStream_t);
+}

@@ -581,9 +581,10 @@ class nonlinear_solver(object):
         J = None
         for k in self._species_loop():
             Jk = self._buf('J', F64, (3, self._Q))
-            _lib.check(self._L.boltx_currents(ctypes.byref(self._grid),
-                                              ctypes.byref(self._phys), _lib.ptr(us[k]),
-                                              _lib.ptr(Jk), _lib.stream_handle()))
+            _lib.check(self._L.boltx_currents_ws(ctypes.byref(self._grid),
+                                                 ctypes.byref(self._phys), _lib.ptr(us[k]),
+                                                 _lib.ptr(Jk), _lib.ptr(self._ws),
+                                                 _lib.stream_handle()))
             if J is None:
                 J = self._spc[0].bufs.setdefault(name, torch.empty_like(Jk))
                 J.copy_(Jk)

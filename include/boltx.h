@@ -206,7 +206,9 @@ int boltx_fill_ghosts(const boltx_grid *grid, const boltx_physics *phys, void *f
 
 /* Bytes of device workspace boltx_fvm_stage and boltx_moments use for this
  * problem (required in the q1-line layout, optional in the reference layout,
- * where it holds the sign-grouped p order), and its one-time set-up.  The
+ * where it holds the sign-grouped p order and, with p-advection in three p
+ * axes, the q-part of L between the stage's two kernels: up to one more
+ * f-sized array, at most 2 GiB), and its one-time set-up.  The
  * reference has no counterpart: ArrayFire allocates its temporaries itself;
  * here the caller owns all device memory. */
 size_t boltx_workspace_size(const boltx_grid *grid, const boltx_physics *phys);
@@ -218,6 +220,12 @@ int boltx_workspace_init(const boltx_grid *grid, const boltx_physics *phys,
  * J3 = charge * mom_v3_bulk(f).  Replaces df_dt_fvm.py:214-224. */
 int boltx_currents(const boltx_grid *grid, const boltx_physics *phys,
                    const void *u, double *J, void *stream);
+
+/* boltx_currents with the workspace of the stage (boltx_workspace_size bytes,
+ * set up by boltx_workspace_init; NULL: as boltx_currents), which holds the
+ * partial sums of the marching kernel.  The same sums in another fixed order. */
+int boltx_currents_ws(const boltx_grid *grid, const boltx_physics *phys,
+                      const void *u, double *J, void *workspace, void *stream);
 
 /* One FDTD leapfrog on the periodic Yee grid, in place on yee ([6][Q] FP64:
  * E1(i,j+1/2), E2(i+1/2,j), E3(i+1/2,j+1/2), B1(i+1/2,j), B2(i,j+1/2),

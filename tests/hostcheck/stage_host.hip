@@ -261,3 +261,41 @@ static int ppm_split_mismatch(const double* y, int n) {
 extern "C" int host_ppm_split_mismatch(int precision, const double* y, int n) {
   return precision == 0 ? ppm_split_mismatch<double>(y, n) : ppm_split_mismatch<float>(y, n);
 }
+
+#include "../../bolt_amd/csrc/dir_recon.h"
+
+// The direction-dependent states (dir_recon.h) on n five-cell windows: the
+// right face of the centre cell (pos) or its left face, from the aux
+// quantities of the three inner cells.
+template <typename T, int R>
+static void dir_states(const double* y, double* out, int n, bool pos) {
+  const DirCoef<T> c = dir_coef<R, T>(pos);
+  for (int i = 0; i < n; ++i) {
+    T a[5];
+    for (int k = 0; k < 5; ++k) a[k] = T(y[5 * i + k]);
+    const T k1 = dir_aux<R, T>(a[0], a[1], a[2]), k2 = dir_aux<R, T>(a[1], a[2], a[3]);
+    const T k3 = dir_aux<R, T>(a[2], a[3], a[4]);
+    out[i] = double(dir_state<R, T>(a[0], a[1], a[2], a[3], a[4], k1, k2, k3, pos, c));
+  }
+}
+
+extern "C" int host_dir_states(int recon, int precision, int pos, const double* y, double* out,
+                               int n) {
+  const bool p = pos != 0;
+  if (precision == 0) {
+    switch (recon) {
+      case 0: dir_states<double, RC_PC>(y, out, n, p); break;
+      case 1: dir_states<double, RC_MINMOD>(y, out, n, p); break;
+      case 2: dir_states<double, RC_PPM>(y, out, n, p); break;
+      default: dir_states<double, RC_WENO5>(y, out, n, p);
+    }
+  } else {
+    switch (recon) {
+      case 0: dir_states<float, RC_PC>(y, out, n, p); break;
+      case 1: dir_states<float, RC_MINMOD>(y, out, n, p); break;
+      case 2: dir_states<float, RC_PPM>(y, out, n, p); break;
+      default: dir_states<float, RC_WENO5>(y, out, n, p);
+    }
+  }
+  return 0;
+}

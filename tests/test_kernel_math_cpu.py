@@ -204,3 +204,31 @@ def test_ppm_split_form_is_bitwise_ppm_faces(precision):
     plain_l = 0.5 * (T5[2] + T5[1])
     assert int((L != plain_l).sum()) > n // 10
     assert lib.host_ppm_split_mismatch(precision, y.ctypes.data, len(y)) == 0
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("recon", [0, 1, 2, 3])
+@pytest.mark.parametrize("pos", [0, 1])
+def test_dir_states_are_the_faces(precision, recon, pos):
+    """The states of dir_recon.h (one per cell, the face chosen per lane) are
+    the q1-line kernels' faces: bit for bit where the arithmetic is the same
+    (all but the order of WENO5's sums and PPM's minima, which are exact),
+    within a few roundings of the largest value for WENO5."""
+    import ctypes
+    from tests.hostcheck import harness as H
+    lib = H.lib()
+    rng = np.random.default_rng(23)
+    n = 20000
+    smooth = 1.0 + 0.3 * rng.standard_normal((n, 5))
+    coarse = np.round(rng.standard_normal((n, 5)) * 2) / 2
+    y = np.ascontiguousarray(np.concatenate([smooth, coarse]))
+    out = [np.empty(len(y)) for _ in range(2)]
+    for name, o in zip(("host_dir_states", "host_ql_faces"), out):
+        fn = getattr(lib, name)
+        fn.argtypes = [ctypes.c_int] * 3 + [ctypes.c_void_p] * 2 + [ctypes.c_int]
+        fn(recon, precision, pos, y.ctypes.data, o.ctypes.data, len(y))
+    if recon == 3:
+        eps = 2.0 ** -52 if precision == 0 else 2.0 ** -23
+        assert np.abs(out[0] - out[1]).max() <= 16 * eps * np.abs(y).max()
+    else:
+        assert np.array_equal(out[0], out[1])

@@ -19,7 +19,7 @@ STEPPER = {"RK2": 0, "SSP-RK3": 1}
 EXPORTS = ("boltx_fvm_stage", "boltx_fvm_stage_noalloc", "boltx_fvm_stage_coeffs",
            "boltx_moments",
            "boltx_workspace_size", "boltx_workspace_init",
-           "boltx_currents", "boltx_currents_ws", "boltx_fdtd_step", "boltx_yee_to_cell_centered",
+           "boltx_currents", "boltx_currents_ws", "boltx_fvm_stage_after_currents", "boltx_fdtd_step", "boltx_yee_to_cell_centered",
            "boltx_check_finite", "boltx_adjoint_stage", "boltx_adjoint_workspace_size",
            "boltx_ensemble_layout", "boltx_ensemble_workspace_size", "boltx_ensemble_map",
            "boltx_ensemble_init", "boltx_ensemble_step", "boltx_fill_ghosts",
@@ -106,6 +106,7 @@ def load(path=LIB_PATH):
     g, ph, st = ctypes.POINTER(Grid), ctypes.POINTER(Physics), ctypes.POINTER(Stage)
     lib.boltx_fvm_stage.argtypes = [g, ph, st, vp]
     lib.boltx_fvm_stage_noalloc.argtypes = [g, ph, st, vp]
+    lib.boltx_fvm_stage_after_currents.argtypes = [g, ph, st, vp]
     lib.boltx_fvm_stage_coeffs.argtypes = [g, ph, st, ctypes.POINTER(Coeffs), vp]
     lib.boltx_moments.argtypes = [g, ph, vp, vp, vp, vp]
     lib.boltx_workspace_size.argtypes = [g, ph]

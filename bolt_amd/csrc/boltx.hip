@@ -806,7 +806,8 @@ static int currents_of(const StageParams& sp, const boltx_physics* phys, double*
 
 // One stage with the given workspace (the caller's, or the scratch array).
 static int fvm_stage_impl(const boltx_grid* grid, const boltx_physics* phys,
-                          const boltx_stage* st, void* workspace, size_t chunk, hipStream_t s) {
+                          const boltx_stage* st, void* workspace, size_t chunk, bool have_D,
+                          hipStream_t s) {
   StageParams sp = base_params(grid);
   sp.riemann_q = phys->riemann_q;
   sp.riemann_p = phys->riemann_p;
@@ -844,9 +845,9 @@ static int fvm_stage_impl(const boltx_grid* grid, const boltx_physics* phys,
     double* part = (double*)(ws + w.o_part);
     if (phys->precision == BOLTX_FP64)
       return psplit_stage<double>(sp, phys->recon_q, phys->recon_p, w.rows, D, part,
-                                  st->currents_out, s);
+                                  st->currents_out, have_D, s);
     return psplit_stage<float>(sp, phys->recon_q, phys->recon_p, w.rows, D, part,
-                               st->currents_out, s);
+                               st->currents_out, have_D, s);
   }
   if (workspace && qc_applies(grid)) {
     // the slab kernels accumulate the currents of u with the moments
@@ -870,7 +871,14 @@ extern "C" int boltx_fvm_stage(const boltx_grid* grid, const boltx_physics* phys
                                const boltx_stage* st, void* stream) {
   int rc = check_stage(grid, phys, st);
   if (rc) return rc;
-  return fvm_stage_impl(grid, phys, st, st->workspace, kSplitChunk, (hipStream_t)stream);
+  return fvm_stage_impl(grid, phys, st, st->workspace, kSplitChunk, false, (hipStream_t)stream);
+}
+
+extern "C" int boltx_fvm_stage_after_currents(const boltx_grid* grid, const boltx_physics* phys,
+                                              const boltx_stage* st, void* stream) {
+  int rc = check_stage(grid, phys, st);
+  if (rc) return rc;
+  return fvm_stage_impl(grid, phys, st, st->workspace, kSplitChunk, true, (hipStream_t)stream);
 }
 
 static Coeff coeff_of(const boltx_coeff& c) {
@@ -1089,7 +1097,7 @@ extern "C" int boltx_fvm_stage_noalloc(const boltx_grid* grid, const boltx_physi
     // the previous call may have left another problem's p order here
     if (grid->layout == BOLTX_LAYOUT_REFERENCE && (rc = init_slab_perm(grid, ws, s))) return rc;
   }
-  return fvm_stage_impl(grid, phys, st, ws, kSplitChunkScratch, s);
+  return fvm_stage_impl(grid, phys, st, ws, kSplitChunkScratch, false, s);
 }
 
 template <typename T>
@@ -1134,11 +1142,12 @@ extern "C" int boltx_currents_ws(const boltx_grid* grid, const boltx_physics* ph
   StageParams sp = base_params(grid);
   sp.u = u;
   sp.charge = phys->charge;
+  void* D = (char*)workspace + w.o_D;
   double* part = (double*)((char*)workspace + w.o_part);
   hipStream_t s = (hipStream_t)stream;
   if (phys->precision == BOLTX_FP64)
-    return psplit_currents<double>(sp, phys->recon_q, w.rows, part, J, s);
-  return psplit_currents<float>(sp, phys->recon_q, w.rows, part, J, s);
+    return psplit_currents<double>(sp, phys->recon_q, w.rows, D, part, J, s);
+  return psplit_currents<float>(sp, phys->recon_q, w.rows, D, part, J, s);
 }
 
 extern "C" int boltx_fdtd_step(const boltx_grid* grid, double* yee, const double* J, double dt,

@@ -3,6 +3,6 @@
 #include "psplit_launch.h"
 
 namespace bx {
-template int psplit_stage<double>(const StageParams&, int, int, int, void*, double*, double*, hipStream_t);
-template int psplit_currents<double>(const StageParams&, int, int, double*, double*, hipStream_t);
+template int psplit_stage<double>(const StageParams&, int, int, int, void*, double*, double*, bool, hipStream_t);
+template int psplit_currents<double>(const StageParams&, int, int, void*, double*, double*, hipStream_t);
 }

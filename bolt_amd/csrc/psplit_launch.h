@@ -11,14 +11,16 @@ namespace bx {
 
 // One stage (sp complete, mom and fields set) over all q2 rows, ``rows`` of
 // them at a time, with D (rows * n_q1 * P values) and, when J is wanted, the
-// partial currents ``part`` (psplit_part_bytes).
+// partial currents ``part`` (psplit_part_bytes).  have_D: D holds the q-part
+// of sp.u already (rows = n_q2).
 template <typename T>
 int psplit_stage(const StageParams& sp, int recon_q, int recon_p, int rows, void* D, double* part,
-                 double* J, hipStream_t s);
+                 double* J, bool have_D, hipStream_t s);
 
-// The currents of sp.u alone.
+// The currents of sp.u; with rows = n_q2 the q-part of sp.u is left in D for
+// the stage that follows.
 template <typename T>
-int psplit_currents(const StageParams& sp, int recon_q, int rows, double* part, double* J,
+int psplit_currents(const StageParams& sp, int recon_q, int rows, void* D, double* part, double* J,
                     hipStream_t s);
 
 inline size_t psplit_part_bytes(const StageParams& sp, int rows) {
@@ -113,7 +115,8 @@ static int pplane_recon(const StageParams& sp, int rp, int r0, int r1, const voi
 
 template <typename T>
 int psplit_stage(const StageParams& sp, int rq, int rp, int rows, void* D, double* part, double* J,
-                 hipStream_t s) {
+                 bool have_D, hipStream_t s) {
+  if (have_D && !J && rows >= sp.n_q2) return pplane_recon<T>(sp, rp, 0, sp.n_q2, D, s);
   for (int r0 = 0; r0 < sp.n_q2; r0 += rows) {
     const int r1 = r0 + rows < sp.n_q2 ? r0 + rows : sp.n_q2;
     int rc = J ? qdiff_recon<T, true, true>(sp, rq, r0, r1, D, part, s)
@@ -126,11 +129,12 @@ int psplit_stage(const StageParams& sp, int rq, int rp, int rows, void* D, doubl
 }
 
 template <typename T>
-int psplit_currents(const StageParams& sp, int rq, int rows, double* part, double* J,
+int psplit_currents(const StageParams& sp, int rq, int rows, void* D, double* part, double* J,
                     hipStream_t s) {
   for (int r0 = 0; r0 < sp.n_q2; r0 += rows) {
     const int r1 = r0 + rows < sp.n_q2 ? r0 + rows : sp.n_q2;
-    int rc = qdiff_recon<T, false, true>(sp, rq, r0, r1, nullptr, part, s);
+    int rc = rows >= sp.n_q2 ? qdiff_recon<T, true, true>(sp, rq, r0, r1, D, part, s)
+                             : qdiff_recon<T, false, true>(sp, rq, r0, r1, nullptr, part, s);
     if (rc) return rc;
     if ((rc = qcur_reduce(sp, r0, r1, part, J, s))) return rc;
   }

@@ -204,6 +204,7 @@ class nonlinear_solver(object):
         self._source = ps.source
         self._initialize(p)
         self._timings = {'time_ts': 0.0, 'steps': 0}
+        self._after_currents = False
         # list of (start, end) HIP events around every stage-kernel call, or None
         self._stage_events = None
 
@@ -605,6 +606,7 @@ class nonlinear_solver(object):
         the fields once with their average J^{n+1/2} and sees the fields at
         n+1; stage 3 sees those at n+1/2."""
         F = [None, None, None]
+        self._after_currents = False  # whether _currents ran on these stage inputs
         if not self._p_adv:
             return F
         fs = self.fields_solver
@@ -617,12 +619,14 @@ class nonlinear_solver(object):
             elif stage == 1:
                 J_n = self._spc[0].bufs['J_n']
                 J_1 = self._currents(us, 'J_1')
+                self._after_currents = True
                 fs.evolve_once_per_step(0.5 * (J_n + J_1), self.dt)
                 fs.stage_fields = fs._cc_at_n
             elif stage == 2:
                 fs.stage_fields = fs._cc_at_n_plus_half
         elif fs.at_n is False:
             fs.evolve_electrodynamic_fields(self._currents(us, 'J_sum'), self.dt)
+            self._after_currents = True
         if self._user_cp:
             # df_dt_fvm.py:251-267: the user's C_p at the p-faces, each call
             # taking the fields through fields_solver.get_fields()
@@ -712,8 +716,10 @@ class nonlinear_solver(object):
         if ev is not None:
             e0 = torch.cuda.Event(enable_timing=True)
             e0.record()
-        _lib.check(self._L.boltx_fvm_stage(ctypes.byref(self._grid), ctypes.byref(self._phys),
-                                           ctypes.byref(st), _lib.stream_handle()))
+        stage = self._L.boltx_fvm_stage_after_currents if self._after_currents else \
+            self._L.boltx_fvm_stage
+        _lib.check(stage(ctypes.byref(self._grid), ctypes.byref(self._phys), ctypes.byref(st),
+                         _lib.stream_handle()))
         if ev is not None:
             e1 = torch.cuda.Event(enable_timing=True)
             e1.record()

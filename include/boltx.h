@@ -223,9 +223,16 @@ int boltx_currents(const boltx_grid *grid, const boltx_physics *phys,
 
 /* boltx_currents with the workspace of the stage (boltx_workspace_size bytes,
  * set up by boltx_workspace_init; NULL: as boltx_currents), which holds the
- * partial sums of the marching kernel.  The same sums in another fixed order. */
+ * partial sums of the marching kernel.  The same sums in another fixed order.
+ * boltx_fvm_stage_after_currents is boltx_fvm_stage for the u this call was
+ * given last with stage->workspace, unchanged since, and with nothing else run
+ * on that workspace in between: the q-fluxes the call evaluated for the
+ * currents are in the workspace and are not evaluated again (where the stage
+ * does not keep them there, it is boltx_fvm_stage).  The same result. */
 int boltx_currents_ws(const boltx_grid *grid, const boltx_physics *phys,
                       const void *u, double *J, void *workspace, void *stream);
+int boltx_fvm_stage_after_currents(const boltx_grid *grid, const boltx_physics *phys,
+                                   const boltx_stage *stage, void *stream);
 
 /* One FDTD leapfrog on the periodic Yee grid, in place on yee ([6][Q] FP64:
  * E1(i,j+1/2), E2(i+1/2,j), E3(i+1/2,j+1/2), B1(i+1/2,j), B2(i,j+1/2),

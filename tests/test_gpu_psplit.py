@@ -89,6 +89,9 @@ def test_split_stage_matches_the_generic_kernel(gpu, nq, np_, recon, form, preci
                                       _lib.ptr(x[0]), _lib.ptr(J), _lib.ptr(s._ws),
                                       _lib.stream_handle()))
     _close(J, ref[2], tol)
+    # the stage that takes the q-fluxes of that call: the same bits
+    for a, b in zip(got[:2], _run(s, "boltx_fvm_stage_after_currents", x, s._ws, False)):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32-bulk"])

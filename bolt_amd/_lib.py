@@ -19,7 +19,8 @@ STEPPER = {"RK2": 0, "SSP-RK3": 1}
 EXPORTS = ("boltx_fvm_stage", "boltx_fvm_stage_noalloc", "boltx_fvm_stage_coeffs",
            "boltx_moments",
            "boltx_workspace_size", "boltx_workspace_init",
-           "boltx_currents", "boltx_currents_ws", "boltx_fvm_stage_after_currents", "boltx_fdtd_step", "boltx_yee_to_cell_centered",
+           "boltx_currents", "boltx_poisson_workspace_size", "boltx_poisson_init", "boltx_poisson",
+           "boltx_currents_ws", "boltx_fvm_stage_after_currents", "boltx_fdtd_step", "boltx_yee_to_cell_centered",
            "boltx_check_finite", "boltx_adjoint_stage", "boltx_adjoint_workspace_size",
            "boltx_ensemble_layout", "boltx_ensemble_workspace_size", "boltx_ensemble_map",
            "boltx_ensemble_init", "boltx_ensemble_step", "boltx_fill_ghosts",
@@ -113,6 +114,9 @@ def load(path=LIB_PATH):
     lib.boltx_workspace_init.argtypes = [g, ph, vp, vp]
     lib.boltx_currents.argtypes = [g, ph, vp, vp, vp]
     lib.boltx_currents_ws.argtypes = [g, ph, vp, vp, vp, vp]
+    lib.boltx_poisson_workspace_size.argtypes = [g]
+    lib.boltx_poisson_init.argtypes = [g, vp, vp]
+    lib.boltx_poisson.argtypes = [g, i32, ctypes.POINTER(vp), ctypes.POINTER(dbl), dbl, vp, vp, vp]
     lib.boltx_fdtd_step.argtypes = [g, vp, vp, dbl, dbl, dbl, vp]
     lib.boltx_yee_to_cell_centered.argtypes = [g, vp, vp, vp]
     lib.boltx_check_finite.argtypes = [g, vp, vp, vp]
@@ -129,6 +133,7 @@ def load(path=LIB_PATH):
     for name in EXPORTS[:-2]:
         getattr(lib, name).restype = ctypes.c_int
     lib.boltx_workspace_size.restype = ctypes.c_size_t
+    lib.boltx_poisson_workspace_size.restype = ctypes.c_size_t
     lib.boltx_adjoint_workspace_size.restype = ctypes.c_size_t
     lib.boltx_ensemble_layout.restype = ctypes.c_longlong
     lib.boltx_ensemble_workspace_size.restype = ctypes.c_size_t

@@ -42,6 +42,7 @@ class fields_solver(object):
         Q = solver.N_q1 * solver.N_q2
         dev = solver.device
         self._yee = torch.zeros(6, Q, dtype=F64, device=dev)
+        self._poisson_ws = None  # workspace of the HIP Poisson solver, made by its first use
         cc = torch.zeros(6, Q, dtype=F64, device=dev)
         self._fdtd = getattr(p, 'fields_solver', 'fdtd').lower() == 'fdtd'
         init = p.fields_initialize
@@ -121,6 +122,27 @@ class fields_solver(object):
     def compute_electrostatic_fields(self, rho):
         """fields.py:559-566; rho is [Q], already summed over species."""
         self._poisson(rho, self._cc)
+
+    def solve_electrostatic(self, moms):
+        """compute_electrostatic_fields from the species' moment blocks: one
+        call of the HIP solver, or the transforms of ``_poisson`` for grids and
+        species counts it does not take."""
+        s = self._solver
+        if self._poisson_ws is None:
+            n = int(s._L.boltx_poisson_workspace_size(ctypes.byref(s._grid)))
+            n = n if len(moms) <= 8 else 0
+            self._poisson_ws = torch.empty(n, dtype=torch.uint8, device=s.device)
+            if n:
+                _lib.check(s._L.boltx_poisson_init(ctypes.byref(s._grid),
+                                                   _lib.ptr(self._poisson_ws),
+                                                   _lib.stream_handle()))
+                self._charges = (ctypes.c_double * len(moms))(*[sp.charge for sp in s._spc])
+        if self._poisson_ws.numel() == 0:
+            return self.compute_electrostatic_fields(s._rho(moms))
+        density = (ctypes.c_void_p * len(moms))(*[m.data_ptr() for m in moms])
+        _lib.check(s._L.boltx_poisson(ctypes.byref(s._grid), len(moms), density, self._charges,
+                                      float(self.params.eps), _lib.ptr(self._cc),
+                                      _lib.ptr(self._poisson_ws), _lib.stream_handle()))
 
     def _cc_to_yee_E(self, cc):
         """fields.py:497-525 for E: E1 at (i, j+1/2) = (E1[i] + E1[i-1]) / 2,

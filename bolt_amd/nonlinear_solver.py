@@ -611,7 +611,7 @@ class nonlinear_solver(object):
             return F
         fs = self.fields_solver
         if self._es:  # df_dt_fvm.py:235-242: rho of the stage input
-            fs.compute_electrostatic_fields(self._rho(self._stage_moms))
+            fs.solve_electrostatic(self._stage_moms)
         elif fs.coupling == 'once-per-step':
             if stage == 0:
                 # J(u^n) comes out of this stage's kernels (_advance sums it)

@@ -234,6 +234,19 @@ int boltx_currents_ws(const boltx_grid *grid, const boltx_physics *phys,
 int boltx_fvm_stage_after_currents(const boltx_grid *grid, const boltx_physics *phys,
                                    const boltx_stage *stage, void *stream);
 
+/* Electrostatic fields E1, E2 (rows 0 and 1 of cc, [6][Q]) of the charge density
+ * sum_s charge[s] * density[s] ([Q] FP64 each, row 0 of a moment block; 1..8
+ * species) on the periodic q grid.  Replaces fft_poisson
+ * (bolt/lib/nonlinear/fields/electrostatic/fft.py:9-78).  The workspace
+ * (boltx_poisson_workspace_size bytes; 0: the grid is beyond what this solver
+ * takes, 4096 cells on one axis, or 512 per axis and n_q1 n_q2 (n_q1 + n_q2) <=
+ * 2^25 on two) is set up once by
+ * boltx_poisson_init; solves that share it must be stream-ordered. */
+size_t boltx_poisson_workspace_size(const boltx_grid *grid);
+int boltx_poisson_init(const boltx_grid *grid, void *workspace, void *stream);
+int boltx_poisson(const boltx_grid *grid, int n_species, const double *const *density,
+                  const double *charge, double eps, double *cc, void *workspace, void *stream);
+
 /* One FDTD leapfrog on the periodic Yee grid, in place on yee ([6][Q] FP64:
  * E1(i,j+1/2), E2(i+1/2,j), E3(i+1/2,j+1/2), B1(i+1/2,j), B2(i,j+1/2),
  * B3(i,j)): E += dt/(mu eps) curl B - dt J / eps, then B -= dt curl E.

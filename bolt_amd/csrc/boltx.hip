@@ -528,14 +528,32 @@ constexpr size_t kSplitChunkScratch = (size_t)40 << 20;
 // Cells from which the two-kernel stage is the faster one.
 constexpr double kSplitCells = 786432;
 
+// Cells from which the marching stage without p-advection is the faster one
+// (whole FP64 steps, slab kernel / march): PPM 0.9 M cells 108 / 99 us, 1.7 M
+// 138 / 128, 6.3 M 422 / 270, 35 M 1874 / 1037; WENO5 1.7 M 144 / 135, 6.3 M
+// 448 / 296; minmod, whose slab kernel does little, 1.7 M 108 / 112, 2.5 M 140 /
+// 140, 6.5 M 228 / 221, 35 M 1399 / 883.
+constexpr double kMarchCells = 1572864, kMarchCellsMinmod = 4194304;
+
 // Workspace of the reference layout: the sign-grouped p order, then (with the
 // two-kernel stage) D and the partial currents.
 struct RefWorkspace {
-  int rows = 0;  // q2 rows per chunk; 0: the two-kernel stage does not apply
-  size_t o_D = 0, o_part = 0, total = 0;
+  int rows = 0;   // q2 rows per chunk; 0: neither of the marching stages applies
+  size_t o_D = 0; // D, or (without p-advection) the Maxwellian factors
+  size_t o_part = 0, total = 0;
 };
 
 static size_t align256(size_t x) { return (x + 255) / 256 * 256; }
+
+// The marching stage without p-advection (qdiff_kernel, QK_STAGE): enough
+// p-cells to fill its waves and enough cells that its three launches per stage
+// beat the one of the slab kernel.  FP32 WENO5 stays with the slab kernel, whose
+// rounding of the weights its results have always had.
+static bool qmarch_applies(const boltx_physics* ph, size_t P, double cells) {
+  if (ph->precision != BOLTX_FP64 && ph->recon_q == RC_WENO5) return false;
+  const bool light = ph->recon_q == RC_PC || ph->recon_q == RC_MINMOD;
+  return P >= 48 && cells >= (light ? kMarchCellsMinmod : kMarchCells);
+}
 
 // The two-kernel stage takes p-advection with a (p1, p2) plane of one
 // workgroup's threads, a row of D that the scratch array holds (both entry
@@ -547,13 +565,23 @@ static RefWorkspace ref_workspace(const boltx_grid* g, const boltx_physics* ph, 
   RefWorkspace w;
   if (!qc_applies(g)) return w;
   w.total = qc_workspace_bytes(qc_nslab(g));
-  if (!ph->p_advection || g->n_p1 < 2 || g->n_p2 < 2 || g->n_p3 < 2 ||
-      (long)g->n_p1 * g->n_p2 > 1024 || g->n_q1 < 2 ||
-      (double)g->n_p1 * g->n_p2 * g->n_p3 * g->n_q1 * g->n_q2 < kSplitCells)
-    return w;
   const size_t P = (size_t)g->n_p1 * g->n_p2 * g->n_p3;
-  const size_t row = P * g->n_q1 * (ph->precision == BOLTX_FP64 ? 8 : 4);
-  const size_t prow = (P + 63) / 64 * 3 * sizeof(double) * g->n_q1;
+  const double cells = (double)P * g->n_q1 * g->n_q2;
+  const size_t esz = ph->precision == BOLTX_FP64 ? 8 : 4, slabs = (P + 63) / 64;
+  if (g->n_q1 < 2) return w;
+  size_t row, prow;  // bytes per q2 row
+  if (ph->p_advection) {
+    if (g->n_p1 < 2 || g->n_p2 < 2 || g->n_p3 < 2 || (long)g->n_p1 * g->n_p2 > 1024 ||
+        cells < kSplitCells)
+      return w;
+    row = P * g->n_q1 * esz;
+    prow = slabs * 3 * sizeof(double) * g->n_q1;
+  } else {
+    if (!qmarch_applies(ph, P, cells)) return w;
+    row = (size_t)(g->n_p1 + g->n_p2 + g->n_p3) * g->n_q1 * esz;
+    prow = slabs * 5 * sizeof(double) * g->n_q1;
+    if (P * g->n_q1 * esz > kSplitChunkScratch) return w;  // 32-bit offsets in a row of q-cells
+  }
   if (row + prow > kSplitChunkScratch) return w;
   const long most = std::max(1L, (long)(chunk / (row + prow)));
   const long nchunk = (g->n_q2 + most - 1) / most;
@@ -837,12 +865,16 @@ static int fvm_stage_impl(const boltx_grid* grid, const boltx_physics* phys,
     if (phys->precision == BOLTX_FP64) return ql_stage<double>(grid, phys, st, workspace, sp, s);
     return ql_stage<float>(grid, phys, st, workspace, sp, s);
   }
-  // (currents of a grid with ghost rows: the slab kernel)
+  // (currents of a grid with ghost rows or without p-advection: the slab kernel)
   if (const RefWorkspace w = ref_workspace(grid, phys, chunk);
-      workspace && w.rows > 0 && !(st->currents_out && ghost_rows(grid) > 0)) {
+      workspace && w.rows > 0 && !(st->currents_out && (ghost_rows(grid) > 0 || !padv))) {
     char* ws = (char*)workspace;
     void* D = ws + w.o_D;
     double* part = (double*)(ws + w.o_part);
+    if (!padv)
+      return phys->precision == BOLTX_FP64
+                 ? qmarch_stage<double>(sp, phys->recon_q, w.rows, D, part, s)
+                 : qmarch_stage<float>(sp, phys->recon_q, w.rows, D, part, s);
     if (phys->precision == BOLTX_FP64)
       return psplit_stage<double>(sp, phys->recon_q, phys->recon_p, w.rows, D, part,
                                   st->currents_out, have_D, s);
@@ -1137,7 +1169,7 @@ extern "C" int boltx_currents_ws(const boltx_grid* grid, const boltx_physics* ph
   if (grid->layout != BOLTX_LAYOUT_REFERENCE)
     return fail(BOLTX_EUNSUPPORTED, "currents need the reference layout");
   const RefWorkspace w = ref_workspace(grid, phys, kSplitChunk);
-  if (!workspace || w.rows == 0 || ghost_rows(grid) > 0)
+  if (!workspace || w.rows == 0 || ghost_rows(grid) > 0 || !phys->p_advection)
     return boltx_currents(grid, phys, u, J, stream);
   StageParams sp = base_params(grid);
   sp.u = u;

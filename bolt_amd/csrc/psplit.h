@@ -40,9 +40,22 @@ struct QDiffParams {
   StageParams sp;
   int r0, r1;                // q2 rows of the chunk
   int nslab, ntile, nseg;    // 64-wide p slabs, groups of 4 q1 tiles, q2 segments of the chunk
-  void* D;                   // [r1 - r0][n_q1][P], or NULL
-  double* part;              // [nslab][3][(r1 - r0) * n_q1] partial currents, or NULL
+  void* D;                   // [r1 - r0][n_q1][P] (QK_DIV)
+  double* part;              // [nslab][3 or 5][(r1 - r0) * n_q1] partial currents or moments
+  const void* tab;           // [r1 - r0][n_q1][n_p1 + n_p2 + n_p3] Maxwellian factors (QK_STAGE)
 };
+
+// What qdiff_kernel produces: currents of u and / or the q-part of L, or the
+// whole stage of a problem without p-advection, with the partial moments of
+// its output (as a separate pass they would read it again).  The last is the
+// slab kernel's work at 2-V sizes: 100 x 75 q x 30 x 28 p, PPM, FP64: 141 us per
+// stage there; here 76 us, 6 for the Maxwellian factors and 5 for the moments.
+// It is bound by its own latency (three waves per SIMD, 2900 waves) and, with
+// scalar registers spilled to vector lanes, by about 190 VALU per cell; reading
+// the stage's arguments again in every row instead made it slower (270 -> 284 us
+// per step).  Two q1 cells per lane in FP64 (270 us per step; four: 316), four in
+// FP32 (206; two: 221).
+enum QDiffKind : int { QK_CUR = 1, QK_DIV = 2, QK_DIV_CUR = 3, QK_STAGE = 4 };
 
 // Sums of x[0..M-1] (M at most 16) over the 64 lanes through the wave's LDS
 // area of M rows: the sum of value lane / 4 is returned in every lane of the
@@ -86,9 +99,11 @@ struct Block {
 };
 
 // GH: one of the q axes has ghost rows (plain addressing of whole rows).
-template <typename T, int R, int N, bool GH, bool DIV, bool CUR>
-__global__ __launch_bounds__(256) void qdiff_kernel(QDiffParams q) {
-  __shared__ double area[CUR ? 4 : 1][CUR ? 3 * N * LS_PITCH : 1];
+template <typename T, int R, int N, bool GH, int KIND>
+__global__ __launch_bounds__(256, (KIND == QK_STAGE ? 3 : 1)) void qdiff_kernel(QDiffParams q) {
+  constexpr bool DIV = (KIND & QK_DIV) != 0, CUR = (KIND & QK_CUR) != 0, STAGE = KIND == QK_STAGE;
+  constexpr int NS = CUR ? 3 : STAGE ? 4 : 0;  // sums per cell taken together
+  __shared__ double area[NS ? 4 : 1][NS ? NS * N * LS_PITCH : 1];
   const StageParams& sp = q.sp;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int nb = gridDim.x;
@@ -111,8 +126,16 @@ __global__ __launch_bounds__(256) void qdiff_kernel(QDiffParams q) {
   const int j23 = fdivmod((int)p, sp.n_p1, 1.0f / float(sp.n_p1), j1);
   const int j3 = fdivmod(j23, sp.n_p2, 1.0f / float(sp.n_p2), j2);
   const double v1 = centre(sp.p1s, j1, sp.dp1), v2 = centre(sp.p2s, j2, sp.dp2);
-  const double v3 = CUR ? centre(sp.p3s, j3, sp.dp3) : 0.0;
+  const double v3 = CUR || STAGE ? centre(sp.p3s, j3, sp.dp3) : 0.0;
   const T C1 = T(v1), C2 = T(v2);
+  // QK_STAGE: energy weight, RK coefficients and the offsets of the lane's
+  // Maxwellian factors in a q-cell's row of the table
+  const double ev = 0.5 * ((v1 * v1 + v2 * v2) + v3 * v3);
+  const T ta = T(sp.a), tb = T(sp.b), tcdt = T(sp.cdt), ttau = T(sp.inv_tau);
+  const bool use_un = sp.a != 0.0, w_is_u = sp.w == sp.u, b_one = sp.b == 1.0;
+  const int TS = sp.n_p1 + sp.n_p2 + sp.n_p3;
+  const unsigned x1 = j1 * (unsigned)sizeof(T), x2 = (sp.n_p1 + j2) * (unsigned)sizeof(T),
+                 x3 = (sp.n_p1 + sp.n_p2 + j3) * (unsigned)sizeof(T);
   const bool pos1 = C1 > T(0), pos2 = C2 > T(0);
   const DirCoef<T> k1 = dir_coef<R, T>(pos1), k2 = dir_coef<R, T>(pos2);
   const T tinv1 = T(sp.inv_dq1), tinv2 = T(sp.inv_dq2);
@@ -280,6 +303,52 @@ __global__ __launch_bounds__(256) void qdiff_kernel(QDiffParams q) {
                      (c0 + k) * (int)(P * (long)sizeof(T)));
       }
     }
+    if constexpr (STAGE) {
+      const long at = (long)r * n1 * P;
+      const Block<T> wr((const T*)sp.w + at, n1 * P), unr((const T*)sp.un + at, n1 * P),
+          outr((const T*)sp.out + at, n1 * P),
+          tr((const T*)q.tab + (long)(r - q.r0) * n1 * TS, (long)n1 * TS);
+      T wv[N], uv[N], fmb[N];
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        const int c = c0 + k < n1 ? c0 + k : n1 - 1;
+        const int o = c * (int)(P * (long)sizeof(T)), to = c * TS * (int)sizeof(T);
+        wv[k] = w_is_u ? f[k] : wr.load(pb, o);
+        uv[k] = use_un ? unr.load(pb, o) : T(0);
+        fmb[k] = T(0);
+        if (sp.source) {
+          fmb[k] = tr.load(x1, to);
+          if (sp.p_dim >= 2) fmb[k] = fmb[k] * tr.load(x2, to);
+          if (sp.p_dim >= 3) fmb[k] = fmb[k] * tr.load(x3, to);
+        }
+      }
+      double x[4 * N], m3[N];
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        T d = ql_fma(-t1[k], tinv1, -(t2[k] * tinv2));
+        if (sp.source) d = ql_fma(fmb[k] - f[k], ttau, d);
+        const T tv = ql_fma(d, tcdt, wv[k]);
+        const T o = use_un ? ql_fma(tb, tv, ta * uv[k]) : (b_one ? tv : tb * tv);
+        if (valid && c0 + k < n1) outr.store(o, pb, (c0 + k) * (int)(P * (long)sizeof(T)));
+        const double od = valid ? double(o) : 0.0;
+        x[4 * k] = od;
+        x[4 * k + 1] = od * v1;
+        x[4 * k + 2] = od * v2;
+        x[4 * k + 3] = od * ev;
+        m3[k] = od * v3;
+      }
+      const int idx = lane / 4, k = idx / 4, comp = idx - 4 * k;
+      const long nq = (long)rows * n1, cell = (long)(r - q.r0) * n1 + c0 + k;
+      const double sum = lane_sums<4 * N>(x, area[wave], lane);
+      if ((lane & 3) == 0 && k < N && c0 + k < n1)
+        q.part[((long)slab * 5 + (comp < 3 ? comp : 4)) * nq + cell] = sum;
+      // mom_v3: of one p3 cell it is the density's multiple
+      if (sp.n_p3 > 1) {
+        const double s3 = lane_sums<N>(m3, area[wave], lane);
+        if ((lane & 3) == 0 && idx < N && c0 + idx < n1)
+          q.part[((long)slab * 5 + 3) * nq + (long)(r - q.r0) * n1 + c0 + idx] = s3;
+      }
+    }
     if constexpr (CUR) {
       double x[3 * N];
 #pragma unroll
@@ -331,6 +400,57 @@ static __global__ __launch_bounds__(256) void qcur_reduce_kernel(const double* p
 #pragma unroll
     for (int s = 0; s < QCUR_SUBS; ++s) x += red[s][ci];
     J[(long)comp * Q + q0 + i] = charge * (x * measure);
+  }
+}
+
+// Maxwellian factors of the chunk's q-cells from the raw moments
+// (collision_operator.py:52-65, 102-116): per q-cell prefactor * e1 (rounded as
+// the other stage kernels round it), e2, e3; a wave per q-cell.
+template <typename T>
+__global__ __launch_bounds__(256) void qtab_kernel(StageParams sp, int q0, int nq, T* tab) {
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (i >= nq) return;
+  const BgkCell b = qcell_bgk(sp, q0 + i);
+  const T pref = T(maxwell_prefactor(b, sp.mass, sp.kB, sp.p_dim));
+  const int TS = sp.n_p1 + sp.n_p2 + sp.n_p3;
+  T* row = tab + (long)i * TS;
+  for (int j = lane; j < TS; j += 64) {
+    const int ax = j < sp.n_p1 ? 0 : j < sp.n_p1 + sp.n_p2 ? 1 : 2;
+    const double v = ax == 0 ? centre(sp.p1s, j, sp.dp1)
+                     : ax == 1 ? centre(sp.p2s, j - sp.n_p1, sp.dp2)
+                               : centre(sp.p3s, j - sp.n_p1 - sp.n_p2, sp.dp3);
+    const T e = T(maxwell_factor(v, ax == 0 ? b.u1 : ax == 1 ? b.u2 : b.u3, b.T, sp.mass, sp.kB));
+    row[j] = ax == 0 ? pref * e : e;
+  }
+}
+
+// Moment blocks of the chunk from the partial moments: 16 threads per q-cell
+// take interleaved slabs, and the 16 sums are added in order.
+static __global__ __launch_bounds__(256) void qmom_reduce_kernel(StageParams sp, const double* part,
+                                                                 int nslab, int nq, int q0) {
+  __shared__ double red[5][QCUR_SUBS][16];
+  const int ci = threadIdx.x & 15, sub = threadIdx.x >> 4;
+  const int i = blockIdx.x * 16 + ci;
+  double a[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  if (i < nq)
+    for (int s = sub; s < nslab; s += QCUR_SUBS)
+#pragma unroll
+      for (int k = 0; k < 5; ++k)
+        if (k != 3 || sp.n_p3 > 1) a[k] += part[((long)s * 5 + k) * nq + i];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) red[k][sub][ci] = a[k];
+  __syncthreads();
+  if (sub == 0 && i < nq) {
+    double m[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      double x = 0.0;
+#pragma unroll
+      for (int s = 0; s < QCUR_SUBS; ++s) x += red[k][s][ci];
+      m[k] = x * sp.measure;
+    }
+    if (sp.n_p3 == 1) m[3] = m[0] * centre(sp.p3s, 0, sp.dp3);
+    write_moment_block(sp.mom_out, sp.Q, q0 + i, m, sp.mass, sp.kB, sp.p_dim);
   }
 }
 

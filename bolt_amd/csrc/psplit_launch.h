@@ -23,16 +23,23 @@ template <typename T>
 int psplit_currents(const StageParams& sp, int recon_q, int rows, void* D, double* part, double* J,
                     hipStream_t s);
 
+// One stage of a problem without p-advection, ``rows`` q2 rows at a time, with
+// the Maxwellian factors ``tab`` (rows * n_q1 * (n_p1 + n_p2 + n_p3) values)
+// and the partial moments ``part``.
+template <typename T>
+int qmarch_stage(const StageParams& sp, int recon_q, int rows, void* tab, double* part,
+                 hipStream_t s);
+
 inline size_t psplit_part_bytes(const StageParams& sp, int rows) {
   return (size_t)((sp.P + 63) / 64) * 3 * (size_t)rows * sp.n_q1 * sizeof(double);
 }
 
 #ifdef BX_PSPLIT_INSTANTIATE
 
-template <typename T, int R, bool DIV, bool CUR>
+template <typename T, int R, int KIND>
 static int qdiff_launch(const StageParams& sp, int r0, int r1, void* D, double* part,
-                        hipStream_t s) {
-  constexpr int N = 4;
+                        const void* tab, hipStream_t s) {
+  constexpr int N = KIND == QK_STAGE && sizeof(T) == 8 ? 2 : 4;
   QDiffParams q;
   q.sp = sp;
   q.r0 = r0;
@@ -46,27 +53,28 @@ static int qdiff_launch(const StageParams& sp, int r0, int r1, void* D, double* 
   q.nseg = nseg;
   q.D = D;
   q.part = part;
+  q.tab = tab;
   const unsigned nb = (unsigned)(q.nslab * q.ntile * nseg);
   if (sp.gh1 || sp.gh2) {
     // (ghost rows occur with electrostatic fields only: no currents)
-    if constexpr (!CUR)
-      hipLaunchKernelGGL((qdiff_kernel<T, R, N, true, DIV, CUR>), dim3(nb), dim3(256), 0, s, q);
+    if constexpr ((KIND & QK_CUR) == 0)
+      hipLaunchKernelGGL((qdiff_kernel<T, R, N, true, KIND>), dim3(nb), dim3(256), 0, s, q);
     else
       return fail(BOLTX_EUNSUPPORTED, "currents of a grid with ghost rows");
   } else {
-    hipLaunchKernelGGL((qdiff_kernel<T, R, N, false, DIV, CUR>), dim3(nb), dim3(256), 0, s, q);
+    hipLaunchKernelGGL((qdiff_kernel<T, R, N, false, KIND>), dim3(nb), dim3(256), 0, s, q);
   }
   return launch_status("qdiff_kernel");
 }
 
-template <typename T, bool DIV, bool CUR>
+template <typename T, int KIND>
 static int qdiff_recon(const StageParams& sp, int rq, int r0, int r1, void* D, double* part,
-                       hipStream_t s) {
+                       const void* tab, hipStream_t s) {
   switch (rq) {
-    case RC_PC: return qdiff_launch<T, RC_PC, DIV, CUR>(sp, r0, r1, D, part, s);
-    case RC_MINMOD: return qdiff_launch<T, RC_MINMOD, DIV, CUR>(sp, r0, r1, D, part, s);
-    case RC_PPM: return qdiff_launch<T, RC_PPM, DIV, CUR>(sp, r0, r1, D, part, s);
-    default: return qdiff_launch<T, RC_WENO5, DIV, CUR>(sp, r0, r1, D, part, s);
+    case RC_PC: return qdiff_launch<T, RC_PC, KIND>(sp, r0, r1, D, part, tab, s);
+    case RC_MINMOD: return qdiff_launch<T, RC_MINMOD, KIND>(sp, r0, r1, D, part, tab, s);
+    case RC_PPM: return qdiff_launch<T, RC_PPM, KIND>(sp, r0, r1, D, part, tab, s);
+    default: return qdiff_launch<T, RC_WENO5, KIND>(sp, r0, r1, D, part, tab, s);
   }
 }
 
@@ -119,8 +127,8 @@ int psplit_stage(const StageParams& sp, int rq, int rp, int rows, void* D, doubl
   if (have_D && !J && rows >= sp.n_q2) return pplane_recon<T>(sp, rp, 0, sp.n_q2, D, s);
   for (int r0 = 0; r0 < sp.n_q2; r0 += rows) {
     const int r1 = r0 + rows < sp.n_q2 ? r0 + rows : sp.n_q2;
-    int rc = J ? qdiff_recon<T, true, true>(sp, rq, r0, r1, D, part, s)
-               : qdiff_recon<T, true, false>(sp, rq, r0, r1, D, nullptr, s);
+    int rc = J ? qdiff_recon<T, QK_DIV_CUR>(sp, rq, r0, r1, D, part, nullptr, s)
+               : qdiff_recon<T, QK_DIV>(sp, rq, r0, r1, D, nullptr, nullptr, s);
     if (rc) return rc;
     if (J && (rc = qcur_reduce(sp, r0, r1, part, J, s))) return rc;
     if ((rc = pplane_recon<T>(sp, rp, r0, r1, D, s))) return rc;
@@ -133,10 +141,31 @@ int psplit_currents(const StageParams& sp, int rq, int rows, void* D, double* pa
                     hipStream_t s) {
   for (int r0 = 0; r0 < sp.n_q2; r0 += rows) {
     const int r1 = r0 + rows < sp.n_q2 ? r0 + rows : sp.n_q2;
-    int rc = rows >= sp.n_q2 ? qdiff_recon<T, true, true>(sp, rq, r0, r1, D, part, s)
-                             : qdiff_recon<T, false, true>(sp, rq, r0, r1, nullptr, part, s);
+    int rc = rows >= sp.n_q2 ? qdiff_recon<T, QK_DIV_CUR>(sp, rq, r0, r1, D, part, nullptr, s)
+                             : qdiff_recon<T, QK_CUR>(sp, rq, r0, r1, nullptr, part, nullptr, s);
     if (rc) return rc;
     if ((rc = qcur_reduce(sp, r0, r1, part, J, s))) return rc;
+  }
+  return 0;
+}
+
+template <typename T>
+int qmarch_stage(const StageParams& sp, int rq, int rows, void* tab, double* part,
+                 hipStream_t s) {
+  for (int r0 = 0; r0 < sp.n_q2; r0 += rows) {
+    const int r1 = r0 + rows < sp.n_q2 ? r0 + rows : sp.n_q2;
+    const int q0 = r0 * sp.n_q1, nq = (r1 - r0) * sp.n_q1;
+    int rc;
+    if (sp.source) {
+      hipLaunchKernelGGL(qtab_kernel<T>, dim3((unsigned)((nq + 3) / 4)), dim3(256), 0, s, sp, q0,
+                         nq, (T*)tab);
+      if ((rc = launch_status("qtab_kernel"))) return rc;
+    }
+    if ((rc = qdiff_recon<T, QK_STAGE>(sp, rq, r0, r1, nullptr, part, tab, s))) return rc;
+    if (!sp.mom_out) continue;
+    hipLaunchKernelGGL(qmom_reduce_kernel, dim3((unsigned)((nq + 15) / 16)), dim3(256), 0, s, sp,
+                       (const double*)part, (sp.P + 63) / 64, nq, q0);
+    if ((rc = launch_status("qmom_reduce_kernel"))) return rc;
   }
   return 0;
 }

@@ -1,5 +1,6 @@
-"""The two-kernel stage with three p axes (psplit.h) and the currents it forms,
-against the generic kernel on random states.
+"""The marching stages (psplit.h), two kernels with three p axes and one without
+p-advection, and the currents the first forms, against the generic kernel on
+random states.
 
 Both evaluate the same formulas; FP64 differs by rounding (the per-RHS bar of
 the parity tests, 1e-12), FP32 by a few roundings of each term (1e-6)."""
@@ -9,7 +10,7 @@ import pytest
 import torch
 
 from bolt_amd import _lib
-from tests.cases import case_2d3v, hip_solver
+from tests.cases import case_2d2v, case_2d3v, hip_solver
 
 pytestmark = pytest.mark.gpu
 
@@ -31,7 +32,8 @@ def _random_stage(s, seed, form):
     def rand(shape, dtype=torch.float64):
         return torch.rand(shape, generator=g, device=s.device, dtype=torch.float64).to(dtype)
 
-    assert s._Q * s._P >= 786432  # where the stage is two kernels
+    # where the marching stages apply: these are the workspaces with room for them
+    assert s._ws.numel() > 16 * s._P + 4096
     u, un, w = (s._alloc_f() for _ in range(3))
     for x in (u, un, w):
         x.copy_(0.5 + rand(x.shape, x.dtype))
@@ -114,3 +116,48 @@ def test_split_stage_in_chunks_is_bitwise_the_same(gpu, precision, nq):
     for a, b in zip(_run(s, "boltx_fvm_stage", x, s._ws, True),
                     _run(s, "boltx_fvm_stage_noalloc", x, None, True)):
         assert torch.equal(a, b)
+
+
+def _fields_off(nq, np_, recon, precision, walls=""):
+    c = case_2d2v(seed=5, N_q=8, N_p=4, N_q1=nq[0], N_q2=nq[1], N_p1=np_[0], N_p2=np_[1],
+                  N_p3=np_[2], recon_q=recon, precision=precision, memory_layout="reference",
+                  p_dim=sum(n > 1 for n in np_))
+    bc = c.boundary_conditions
+    if "1" in walls:
+        bc.in_q1_left = bc.in_q1_right = "mirror"
+    if "2" in walls:
+        bc.in_q2_bottom = bc.in_q2_top = "mirror"
+    return hip_solver(c)
+
+
+@pytest.mark.parametrize("nq,np_,recon,form,walls", [
+    ((101, 75), (30, 28, 1), "ppm", "combine", ""),
+    ((64, 67), (24, 24, 1), "weno5", "first", ""),
+    ((3, 5), (500, 600, 1), "minmod", "midpoint", ""),
+    ((2051, 1), (32, 65, 1), "piecewise-constant", "general", ""),
+    ((33, 34), (12, 11, 13), "ppm", "general", ""),
+    ((50, 47), (27, 27, 1), "weno5", "combine", "1"),
+    ((47, 50), (27, 27, 1), "ppm", "first", "2"),
+    ((45, 51), (30, 26, 1), "weno5", "midpoint", "12"),
+])
+@pytest.mark.parametrize("precision", ["fp64", "fp32-bulk"])
+def test_marching_stage_matches_the_generic_kernel(gpu, nq, np_, recon, form, walls, precision):
+    if precision != "fp64" and recon == "weno5":
+        pytest.skip("FP32 WENO5 keeps the slab kernel")
+    s = _fields_off(nq, np_, recon, precision, walls)
+    x = _random_stage(s, 11, form)
+    for r, o in zip(_run(s, "boltx_fvm_stage", x, None, False)[:2],
+                    _run(s, "boltx_fvm_stage", x, s._ws, False)[:2]):
+        _close(o, r, 1e-12 if precision == "fp64" else 1e-6)
+
+
+def test_marching_stage_in_chunks_is_bitwise_the_same(gpu):
+    s = _fields_off((300, 200), (16, 16, 1), "ppm", "fp64")
+    need = 300 * 200 * (33 * 8 + 4 * 5 * 8)
+    s2 = _fields_off((900, 200), (16, 16, 1), "ppm", "fp64")
+    for sv, chunks in ((s, need > 40 << 20), (s2, 3 * need > 40 << 20)):
+        x = _random_stage(sv, 12, "combine")
+        for a, b in zip(_run(sv, "boltx_fvm_stage", x, sv._ws, False)[:2],
+                        _run(sv, "boltx_fvm_stage_noalloc", x, None, False)[:2]):
+            assert torch.equal(a, b)
+    assert chunks

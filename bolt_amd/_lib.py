@@ -20,6 +20,7 @@ EXPORTS = ("boltx_fvm_stage", "boltx_fvm_stage_noalloc", "boltx_fvm_stage_coeffs
            "boltx_moments",
            "boltx_workspace_size", "boltx_workspace_init",
            "boltx_currents", "boltx_poisson_workspace_size", "boltx_poisson_init", "boltx_poisson",
+           "boltx_advance",
            "boltx_currents_ws", "boltx_fvm_stage_after_currents", "boltx_fdtd_step", "boltx_yee_to_cell_centered",
            "boltx_check_finite", "boltx_adjoint_stage", "boltx_adjoint_workspace_size",
            "boltx_ensemble_layout", "boltx_ensemble_workspace_size", "boltx_ensemble_map",
@@ -81,6 +82,12 @@ class EnsMember(ctypes.Structure):
     _fields_ = [("grid", Grid), ("phys", Physics), ("dt", ctypes.c_double)]
 
 
+class State(ctypes.Structure):
+    """boltx_state: one species of boltx_advance."""
+    _fields_ = [("grid", ctypes.POINTER(Grid)), ("phys", ctypes.POINTER(Physics))] + \
+        [(n, ctypes.c_void_p) for n in ("f", "u1", "u2", "mom", "m1", "m2", "workspace")]
+
+
 class EnsTuning(ctypes.Structure):
     _fields_ = [("chunk_cells", ctypes.c_int32), ("batch_cells", ctypes.c_int32)]
 
@@ -117,6 +124,7 @@ def load(path=LIB_PATH):
     lib.boltx_poisson_workspace_size.argtypes = [g]
     lib.boltx_poisson_init.argtypes = [g, vp, vp]
     lib.boltx_poisson.argtypes = [g, i32, ctypes.POINTER(vp), ctypes.POINTER(dbl), dbl, vp, vp, vp]
+    lib.boltx_advance.argtypes = [i32, ctypes.POINTER(State), i32, dbl, dbl, vp, vp, vp, vp]
     lib.boltx_fdtd_step.argtypes = [g, vp, vp, dbl, dbl, dbl, vp]
     lib.boltx_yee_to_cell_centered.argtypes = [g, vp, vp, vp]
     lib.boltx_check_finite.argtypes = [g, vp, vp, vp]

@@ -137,7 +137,7 @@ __global__ __launch_bounds__(kBlock) void fvm_stage_kernel(StageParams sp) {
     block_sum(acc, red);
     if (threadIdx.x == 0) {
       for (int k = 0; k < 5; ++k) acc[k] *= sp.measure;
-      write_moment_block(sp.mom_out, sp.Q, q, acc, sp.mass, sp.kB, sp.p_dim);
+      finish_moments(sp, q, acc);
     }
   }
 }
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(kBlock) void moments_kernel(StageParams sp) {
   block_sum(acc, red);
   if (threadIdx.x == 0) {
     for (int k = 0; k < 5; ++k) acc[k] *= sp.measure;
-    write_moment_block(sp.mom_out, sp.Q, q, acc, sp.mass, sp.kB, sp.p_dim);
+    finish_moments(sp, q, acc);
   }
 }
 
@@ -702,7 +702,7 @@ static size_t ql_workspace_bytes(const boltx_grid* g, int precision) {
 
 template <typename T>
 static int ql_moments(const boltx_grid* g, const StageParams& sp, const void* f, double* mom,
-                      double* part, hipStream_t s) {
+                      double* part, T* next_tab, hipStream_t s) {
   if (mline_vec_applies<T>(g->n_q1)) {
     hipLaunchKernelGGL(mline_vec_kernel<T>, dim3(g->n_q2 * ML_CHUNKS), dim3(256), 0, s,
                        (const T*)f, g->n_q1, g->n_q2, sp.P, ML_CHUNKS, g->n_p1, g->n_p2,
@@ -715,22 +715,40 @@ static int ql_moments(const boltx_grid* g, const StageParams& sp, const void* f,
   }
   int rc = launch_status("mline_kernel");
   if (rc) return rc;
+  if (next_tab) {
+    hipLaunchKernelGGL(ml_finalize_tables_kernel<T>, dim3((sp.Q + 15) / 16), dim3(256), 0, s, part,
+                       ML_CHUNKS, sp.Q, sp.measure, mom, sp.mass, sp.kB, sp.p_dim, sp.flag,
+                       g->n_p1, g->n_p2, g->n_p3, g->p1_start, g->dp1, g->p2_start, g->dp2,
+                       g->p3_start, g->dp3, next_tab);
+    return launch_status("ml_finalize_tables_kernel");
+  }
   // one wave per workgroup: Q threads spread over every CU
   hipLaunchKernelGGL(ml_finalize_kernel, dim3((sp.Q + 63) / 64), dim3(64), 0, s, part,
-                     ML_CHUNKS, sp.Q, sp.measure, mom, sp.mass, sp.kB, sp.p_dim);
+                     ML_CHUNKS, sp.Q, sp.measure, mom, sp.mass, sp.kB, sp.p_dim, sp.flag);
   return launch_status("ml_finalize_kernel");
 }
 
+// What a stage's callers know beyond its arguments.
+struct StageContext {
+  size_t chunk = kSplitChunk;  // bytes of D per chunk
+  bool have_D = false;         // the workspace holds the q-part of u (psplit_stage)
+  int* flag = nullptr;         // divergence flag of the output
+  // q1-line layout: the workspace holds the Maxwellian tables of u already; the
+  // tables of the output are to be left there for the stage that follows
+  bool have_tables = false, next_tables = false;
+};
+
 template <typename T>
 static int ql_stage(const boltx_grid* g, const boltx_physics* ph, const boltx_stage* st,
-                    void* workspace, const StageParams& sp, hipStream_t s) {
+                    void* workspace, const StageParams& sp, const StageContext& cx,
+                    hipStream_t s) {
   if (g->n_q1 > 1 && g->n_q1 < QL_HALO)
     return fail(BOLTX_EUNSUPPORTED, "the q1-line layout needs n_q1 = 1 or n_q1 >= %d", QL_HALO);
   char* ws = (char*)workspace;
   T* tab = (T*)ws;
   double* part = (double*)(ws + ql_table_bytes(g, ph->precision));
   int rc;
-  if (sp.source) {
+  if (sp.source && !cx.have_tables) {
     const dim3 tg((unsigned)((sp.Q + 255) / 256), (unsigned)(g->n_p1 + g->n_p2 + g->n_p3));
     hipLaunchKernelGGL(bgk_table_kernel<T>, tg, dim3(256), 0, s,
                        st->mom_in, sp.Q, g->n_p1, g->n_p2, g->n_p3, g->p1_start, g->dp1,
@@ -774,7 +792,9 @@ static int ql_stage(const boltx_grid* g, const boltx_physics* ph, const boltx_st
   const int nb = (int)(groups * q.nseg);
   ql_launch<T>(q, ph->recon_q, nb, mode, pd, s);
   if ((rc = launch_status("qline_kernel"))) return rc;
-  if (st->mom_out) return ql_moments<T>(g, sp, st->out, st->mom_out, part, s);
+  if (st->mom_out)
+    return ql_moments<T>(g, sp, st->out, st->mom_out, part,
+                         cx.next_tables && sp.source ? tab : nullptr, s);
   return BOLTX_OK;
 }
 
@@ -834,9 +854,10 @@ static int currents_of(const StageParams& sp, const boltx_physics* phys, double*
 
 // One stage with the given workspace (the caller's, or the scratch array).
 static int fvm_stage_impl(const boltx_grid* grid, const boltx_physics* phys,
-                          const boltx_stage* st, void* workspace, size_t chunk, bool have_D,
+                          const boltx_stage* st, void* workspace, const StageContext& cx,
                           hipStream_t s) {
   StageParams sp = base_params(grid);
+  sp.flag = cx.flag;
   sp.riemann_q = phys->riemann_q;
   sp.riemann_p = phys->riemann_p;
   sp.source = phys->source_enabled;
@@ -862,11 +883,12 @@ static int fvm_stage_impl(const boltx_grid* grid, const boltx_physics* phys,
   if (grid->layout == BOLTX_LAYOUT_Q1_LINES) {
     if (padv) return fail(BOLTX_EUNSUPPORTED, "p-advection needs the reference layout");
     if (!workspace) return fail(BOLTX_EINVAL, "the q1-line layout needs the workspace");
-    if (phys->precision == BOLTX_FP64) return ql_stage<double>(grid, phys, st, workspace, sp, s);
-    return ql_stage<float>(grid, phys, st, workspace, sp, s);
+    if (phys->precision == BOLTX_FP64)
+      return ql_stage<double>(grid, phys, st, workspace, sp, cx, s);
+    return ql_stage<float>(grid, phys, st, workspace, sp, cx, s);
   }
   // (currents of a grid with ghost rows or without p-advection: the slab kernel)
-  if (const RefWorkspace w = ref_workspace(grid, phys, chunk);
+  if (const RefWorkspace w = ref_workspace(grid, phys, cx.chunk);
       workspace && w.rows > 0 && !(st->currents_out && (ghost_rows(grid) > 0 || !padv))) {
     char* ws = (char*)workspace;
     void* D = ws + w.o_D;
@@ -877,9 +899,9 @@ static int fvm_stage_impl(const boltx_grid* grid, const boltx_physics* phys,
                  : qmarch_stage<float>(sp, phys->recon_q, w.rows, D, part, s);
     if (phys->precision == BOLTX_FP64)
       return psplit_stage<double>(sp, phys->recon_q, phys->recon_p, w.rows, D, part,
-                                  st->currents_out, have_D, s);
+                                  st->currents_out, cx.have_D, s);
     return psplit_stage<float>(sp, phys->recon_q, phys->recon_p, w.rows, D, part,
-                               st->currents_out, have_D, s);
+                               st->currents_out, cx.have_D, s);
   }
   if (workspace && qc_applies(grid)) {
     // the slab kernels accumulate the currents of u with the moments
@@ -903,14 +925,16 @@ extern "C" int boltx_fvm_stage(const boltx_grid* grid, const boltx_physics* phys
                                const boltx_stage* st, void* stream) {
   int rc = check_stage(grid, phys, st);
   if (rc) return rc;
-  return fvm_stage_impl(grid, phys, st, st->workspace, kSplitChunk, false, (hipStream_t)stream);
+  return fvm_stage_impl(grid, phys, st, st->workspace, StageContext(), (hipStream_t)stream);
 }
 
 extern "C" int boltx_fvm_stage_after_currents(const boltx_grid* grid, const boltx_physics* phys,
                                               const boltx_stage* st, void* stream) {
   int rc = check_stage(grid, phys, st);
   if (rc) return rc;
-  return fvm_stage_impl(grid, phys, st, st->workspace, kSplitChunk, true, (hipStream_t)stream);
+  StageContext cx;
+  cx.have_D = true;
+  return fvm_stage_impl(grid, phys, st, st->workspace, cx, (hipStream_t)stream);
 }
 
 static Coeff coeff_of(const boltx_coeff& c) {
@@ -1001,8 +1025,8 @@ extern "C" int boltx_moments(const boltx_grid* grid, const boltx_physics* phys, 
   if (grid->layout == BOLTX_LAYOUT_Q1_LINES) {
     if (!workspace) return fail(BOLTX_EINVAL, "the q1-line layout needs the workspace");
     double* part = (double*)((char*)workspace + ql_table_bytes(grid, phys->precision));
-    if (phys->precision == BOLTX_FP64) return ql_moments<double>(grid, sp, f, mom, part, s);
-    return ql_moments<float>(grid, sp, f, mom, part, s);
+    if (phys->precision == BOLTX_FP64) return ql_moments<double>(grid, sp, f, mom, part, nullptr, s);
+    return ql_moments<float>(grid, sp, f, mom, part, nullptr, s);
   }
   if (phys->precision == BOLTX_FP64)
     hipLaunchKernelGGL(moments_kernel<double>, dim3(sp.Q), dim3(kBlock), 0, s, sp);
@@ -1129,7 +1153,9 @@ extern "C" int boltx_fvm_stage_noalloc(const boltx_grid* grid, const boltx_physi
     // the previous call may have left another problem's p order here
     if (grid->layout == BOLTX_LAYOUT_REFERENCE && (rc = init_slab_perm(grid, ws, s))) return rc;
   }
-  return fvm_stage_impl(grid, phys, st, ws, kSplitChunkScratch, false, s);
+  StageContext cx;
+  cx.chunk = kSplitChunkScratch;
+  return fvm_stage_impl(grid, phys, st, ws, cx, s);
 }
 
 template <typename T>
@@ -1219,6 +1245,95 @@ extern "C" int boltx_check_finite(const boltx_grid* grid, const double* mom, int
   hipLaunchKernelGGL(check_finite_kernel, dim3((Q + 255) / 256), dim3(256), 0, (hipStream_t)stream,
                      mom, Q, flag);
   return launch_status("check_finite_kernel");
+}
+
+// ---- whole steps ----------------------------------------------------------------
+extern "C" int boltx_advance(int n, const boltx_state* sp, int stepper, double dt, double eps,
+                             double* cc, void* poisson_workspace, int32_t* flag, void* stream) {
+  if (n < 1 || !sp) return fail(BOLTX_EINVAL, "advance: no species");
+  if (stepper != BOLTX_RK2 && stepper != BOLTX_SSP_RK3)
+    return fail(BOLTX_EINVAL, "advance: stepper %d", stepper);
+  const int stages = stepper == BOLTX_RK2 ? 2 : 3;
+  if (!sp[0].phys) return fail(BOLTX_EINVAL, "physics is NULL");
+  const bool fields = sp[0].phys->p_advection != 0;
+  if (fields && n > 8) return fail(BOLTX_EUNSUPPORTED, "advance: %d species with fields", n);
+  // stage k of species i (fvm_operator.py:25-33; SSP-RK3)
+  auto plan = [&](int i, int k) {
+    const boltx_state& x = sp[i];
+    boltx_stage st;
+    memset(&st, 0, sizeof(st));
+    st.workspace = x.workspace;
+    st.fields_c_p1 = st.fields_c_p2 = st.fields_c_p3 = cc;
+    st.b = 1.0;
+    st.cdt = dt;
+    const bool last = k == stages - 1;
+    if (k == 0) {
+      st.u = st.w = x.f;
+      st.out = x.u1;
+      if (stepper == BOLTX_RK2) st.cdt = dt / 2;
+    } else if (stepper == BOLTX_RK2) {
+      st.u = x.u1;
+      st.w = x.f;
+      st.out = x.f;
+    } else {
+      st.u = st.w = k == 1 ? x.u1 : x.u2;
+      st.un = x.f;
+      st.out = k == 1 ? x.u2 : x.f;
+      st.a = k == 1 ? 0.75 : 1.0 / 3.0;
+      st.b = k == 1 ? 0.25 : 2.0 / 3.0;
+    }
+    st.mom_in = k == 0 ? x.mom : k == 1 ? x.m1 : x.m2;
+    st.mom_out = last ? x.mom : k == 0 ? x.m1 : x.m2;
+    return st;
+  };
+  int rc;
+  // every argument is checked before the first launch
+  for (int i = 0; i < n; ++i) {
+    if (!sp[i].mom || !sp[i].m1 || (stages == 3 && !sp[i].m2))
+      return fail(BOLTX_EINVAL, "advance: moment blocks missing");
+    for (int k = 0; k < stages; ++k) {
+      const boltx_stage st = plan(i, k);
+      if ((rc = check_stage(sp[i].grid, sp[i].phys, &st))) return rc;
+    }
+    if (ghost_rows(sp[i].grid) > 0)
+      for (int k = 0; k < 4; ++k)
+        if (sp[i].grid->bc[k] == BOLTX_BC_DIRICHLET || sp[i].grid->bc[k] == BOLTX_BC_MIRROR_DIRICHLET)
+          return fail(BOLTX_EUNSUPPORTED, "advance: dirichlet boundaries need their values");
+    if ((sp[i].phys->p_advection != 0) != fields)
+      return fail(BOLTX_EINVAL, "advance: species disagree on p_advection");
+    if (sp[i].grid->n_q1 != sp[0].grid->n_q1 || sp[i].grid->n_q2 != sp[0].grid->n_q2)
+      return fail(BOLTX_EINVAL, "advance: species disagree on the q grid");
+    for (int j = 0; j < i; ++j)
+      if (sp[i].workspace && sp[i].workspace == sp[j].workspace)
+        return fail(BOLTX_EINVAL, "advance: every species needs a workspace of its own");
+  }
+  if (fields && (!cc || !poisson_workspace))
+    return fail(BOLTX_EINVAL, "advance: fields or their workspace are NULL");
+  hipStream_t s = (hipStream_t)stream;
+  for (int k = 0; k < stages; ++k) {
+    if (fields) {
+      const double* density[8];
+      double charge[8];
+      for (int i = 0; i < n; ++i) {
+        density[i] = plan(i, k).mom_in;
+        charge[i] = sp[i].phys->charge;
+      }
+      if ((rc = boltx_poisson(sp[0].grid, n, density, charge, eps, cc, poisson_workspace, stream)))
+        return rc;
+    }
+    for (int i = 0; i < n; ++i) {
+      const boltx_stage st = plan(i, k);
+      if (ghost_rows(sp[i].grid) > 0 &&
+          (rc = boltx_fill_ghosts(sp[i].grid, sp[i].phys, (void*)st.u, nullptr, stream)))
+        return rc;
+      StageContext cx;
+      cx.have_tables = k > 0;
+      cx.next_tables = k < stages - 1;
+      if (k == stages - 1) cx.flag = flag;
+      if ((rc = fvm_stage_impl(sp[i].grid, sp[i].phys, &st, st.workspace, cx, s))) return rc;
+    }
+  }
+  return BOLTX_OK;
 }
 
 // ---- adjoint stage -----------------------------------------------------------

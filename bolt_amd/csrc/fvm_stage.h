@@ -53,6 +53,8 @@ struct StageParams {
   // [3][Q] currents of u (charge * mom_v1(f_left), mom_v2(f_bot), mom_v3(f)),
   // accumulated by the slab kernels, or NULL
   double* Jout;
+  // set to 1 if a density of mom_out is not finite, or NULL
+  int* flag;
 };
 
 // Per-q-cell state the stage needs besides f: the stencil neighbours of the
@@ -100,6 +102,13 @@ __host__ __device__ inline void qcell_neighbours(const StageParams& sp, int q, Q
     c.nb1[k] = q_row_1(sp, i1 + k - 3, i2);
     c.nb2[k] = q_row_2(sp, i1, i2 + k - 3);
   }
+}
+
+// The moment block of q-cell q from its five moments, and the divergence flag
+// (timestep.py:28-38).
+__host__ __device__ inline void finish_moments(const StageParams& sp, int q, const double m[5]) {
+  write_moment_block(sp.mom_out, sp.Q, q, m, sp.mass, sp.kB, sp.p_dim);
+  if (sp.flag && !(m[0] - m[0] == 0.0)) *sp.flag = 1;
 }
 
 // Fields at cell q for the three C_p evaluations, advection_terms.py:179-186.

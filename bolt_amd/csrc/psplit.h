@@ -450,7 +450,7 @@ static __global__ __launch_bounds__(256) void qmom_reduce_kernel(StageParams sp,
       m[k] = x * sp.measure;
     }
     if (sp.n_p3 == 1) m[3] = m[0] * centre(sp.p3s, 0, sp.dp3);
-    write_moment_block(sp.mom_out, sp.Q, q0 + i, m, sp.mass, sp.kB, sp.p_dim);
+    finish_moments(sp, q0 + i, m);
   }
 }
 
@@ -719,7 +719,7 @@ __global__ __launch_bounds__(NT, WAVES) void pplane_kernel(StageParams sp, const
       for (int w = 1; w < NB / 64; ++w) x += red[k][w];
       m[k] = x * sp.measure;
     }
-    write_moment_block(sp.mom_out, sp.Q, q, m, sp.mass, sp.kB, sp.p_dim);
+    finish_moments(sp, q, m);
   }
 }
 

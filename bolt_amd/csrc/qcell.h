@@ -170,7 +170,7 @@ __device__ inline void qc_finish(const StageParams& sp, int q, double (&acc)[5],
       for (int w = 1; w < NW; ++w) x += red[k][w];
       m[k] = x * sp.measure;
     }
-    if (mom) write_moment_block(sp.mom_out, sp.Q, q, m, sp.mass, sp.kB, sp.p_dim);
+    if (mom) finish_moments(sp, q, m);
     if (cur)
       for (int k = 0; k < 3; ++k) sp.Jout[k * sp.Q + q] = sp.charge * m[5 + k];
   }

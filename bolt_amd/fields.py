@@ -123,21 +123,27 @@ class fields_solver(object):
         """fields.py:559-566; rho is [Q], already summed over species."""
         self._poisson(rho, self._cc)
 
-    def solve_electrostatic(self, moms):
-        """compute_electrostatic_fields from the species' moment blocks: one
-        call of the HIP solver, or the transforms of ``_poisson`` for grids and
-        species counts it does not take."""
+    def native_poisson(self):
+        """Whether the HIP solver takes this grid and number of species; its
+        workspace is made by the first call."""
         s = self._solver
         if self._poisson_ws is None:
             n = int(s._L.boltx_poisson_workspace_size(ctypes.byref(s._grid)))
-            n = n if len(moms) <= 8 else 0
+            n = n if len(s._spc) <= 8 else 0
             self._poisson_ws = torch.empty(n, dtype=torch.uint8, device=s.device)
             if n:
                 _lib.check(s._L.boltx_poisson_init(ctypes.byref(s._grid),
                                                    _lib.ptr(self._poisson_ws),
                                                    _lib.stream_handle()))
-                self._charges = (ctypes.c_double * len(moms))(*[sp.charge for sp in s._spc])
-        if self._poisson_ws.numel() == 0:
+                self._charges = (ctypes.c_double * len(s._spc))(*[sp.charge for sp in s._spc])
+        return self._poisson_ws.numel() > 0
+
+    def solve_electrostatic(self, moms):
+        """compute_electrostatic_fields from the species' moment blocks: one
+        call of the HIP solver, or the transforms of ``_poisson`` for grids and
+        species counts it does not take."""
+        s = self._solver
+        if not self.native_poisson():
             return self.compute_electrostatic_fields(s._rho(moms))
         density = (ctypes.c_void_p * len(moms))(*[m.data_ptr() for m in moms])
         _lib.check(s._L.boltx_poisson(ctypes.byref(s._grid), len(moms), density, self._charges,

@@ -742,6 +742,9 @@ class nonlinear_solver(object):
         flag is still set; see strang_timestep).  Each stage evaluates the
         fields once from every species, then runs every species' stage."""
         self.dt = dt
+        if self._advance_native(dt):
+            self.time_elapsed += dt
+            return
         if self._stepper == 'RK2':
             # fvm_operator.py:25-33
             plan = [('f', 'f', None, 'u1', 0.0, 1.0, dt / 2, 'mom', 'm1'),
@@ -789,6 +792,39 @@ class nonlinear_solver(object):
         if self.fields_solver is not None:
             self.fields_solver.stage_fields = None
         self.time_elapsed += dt
+
+    def _advance_native(self, dt):
+        """The whole step as one call of the library, where the host has no
+        part in its stages: built-in terms, no values from boundary functions,
+        fields off or the electrostatic ones of the HIP solver, and no events
+        around the stages.  False where _advance has to issue them."""
+        if self._general or self._stage_events is not None or 2 in self._bc or 3 in self._bc:
+            return False
+        es = self._p_adv and self._es and self.fields_solver.native_poisson()
+        if self._p_adv and not es:
+            return False
+        two = self._stepper != 'RK2'
+        states = (_lib.State * len(self._spc))()
+        for k in self._species_loop():
+            x, sp = states[k], self._spc[k]
+            x.grid, x.phys = ctypes.pointer(sp.grid), ctypes.pointer(sp.phys)
+            x.f, x.mom, x.workspace = _lib.ptr(sp.f), _lib.ptr(sp.mom), _lib.ptr(sp.ws)
+            x.u1 = _lib.ptr(self._buf('u1'))
+            x.m1 = _lib.ptr(self._buf('m1', F64, (_lib.MOM_ROWS, self._Q)))
+            if two:
+                x.u2 = _lib.ptr(self._buf('u2'))
+                x.m2 = _lib.ptr(self._buf('m2', F64, (_lib.MOM_ROWS, self._Q)))
+        fs = self.fields_solver if es else None
+        _lib.check(self._L.boltx_advance(
+            len(self._spc), states, _lib.STEPPER[self._stepper], float(dt),
+            float(self.params.eps) if es else 1.0, _lib.ptr(fs._cc) if es else None,
+            _lib.ptr(fs._poisson_ws) if es else None, _lib.ptr(self._flag),
+            _lib.stream_handle()))
+        if es:
+            self._after_currents = False
+            for _ in range(9 if two else 6):
+                fs._take_for_C_p()  # (the time-level toggle of every C_p)
+        return True
 
     def capture(self, n_steps, dt):
         """Record ``n_steps`` steps of ``dt`` (the launches strang_timestep

@@ -265,6 +265,26 @@ int boltx_yee_to_cell_centered(const boltx_grid *grid, const double *yee,
 int boltx_check_finite(const boltx_grid *grid, const double *mom, int32_t *flag,
                        void *stream);
 
+/* One whole step of n species (timestep_fvm, fvm_operator.py:6-50, with the
+ * built-in terms): every stage of every species, mirror ghost rows refilled
+ * before each and, with p_advection, the electrostatic fields of each stage's
+ * input (boltx_poisson into cc, the fields of all three C_p).  f is advanced in
+ * place, mom (its moment block) read and rewritten; u1, u2, m1, m2 are scratch
+ * (u2 and m2 unused by RK2).  *flag (or NULL) is set to 1 if a
+ * density of the result is not finite.  The same launches as the stage calls,
+ * and fewer: what one stage of the step prepares for the next stays in the
+ * workspace.  Everything is checked before the first launch. */
+typedef struct boltx_state {
+  const boltx_grid *grid;
+  const boltx_physics *phys;
+  void *f, *u1, *u2;
+  double *mom, *m1, *m2;
+  void *workspace;
+} boltx_state;
+
+int boltx_advance(int n, const boltx_state *species, int stepper, double dt, double eps,
+                  double *cc, void *poisson_workspace, int32_t *flag, void *stream);
+
 /* Adjoint of one stage (FP64, fields off, periodic q: a grid with ghost
  * q-rows is rejected with BOLTX_EUNSUPPORTED).  For the stage
  * out = a*un + b*(w + cdt*L(u)) and an adjoint lam of its output, the caller

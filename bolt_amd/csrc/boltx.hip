@@ -658,6 +658,13 @@ constexpr int ML_CHUNKS = 8;
 // segments 0.740 ms per FP64 step, 8 segments 0.752, 2 segments 0.782, 6
 // (uneven) 0.764; FP32-bulk 0.383-0.386 for 4 and 8.  BOLTX_QL_SEGMENTS
 // overrides the count (tuning sweeps).
+// At most kLineBlocks workgroups per CU count as slots, also where more are
+// resident: with one wave of each per SIMD the march is bound by VALU issue, and
+// shorter segments only repeat the window rows (64^2 q with 24^2 p, FP32-bulk
+// graph replay, 16 -> 8 segments: 78.4 -> 75.7 us; 64^2 q with 32^2 p, FP64
+// adjoint of 10 steps, 8 -> 4: 5.32 -> 5.08 ms).
+constexpr int kLineBlocks = 4;
+
 static int ql_segments(int n2, long groups, long slots) {
   if (const char* e = getenv("BOLTX_QL_SEGMENTS")) {
     const int v = atoi(e);
@@ -672,20 +679,20 @@ static int ql_segments(int n2, long groups, long slots) {
 // Resident q1-line workgroups on the current device for the kernel picked
 // by (precision, n1, recon, mode, pd), cached per device and kernel.
 template <typename T>
-static long ql_slots(int n1, int recon, int mode, int pd) {
+static long ql_slots(int n1, bool rot, int recon, int mode, int pd) {
   static std::mutex mu;
-  static std::map<std::array<int, 5>, long> cache;
+  static std::map<std::array<int, 6>, long> cache;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 0;
   const int nrc = n1 <= 64 ? 1 : n1 <= 128 ? 2 : 4;
-  const std::array<int, 5> key{dev, nrc, recon, mode, pd};
+  const std::array<int, 6> key{dev, nrc, rot, recon, mode, pd};
   std::lock_guard<std::mutex> lock(mu);
   auto it = cache.find(key);
   if (it != cache.end()) return it->second;
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     cus = 0;
-  const long v = (long)cus * ql_blocks_per_cu<T>(n1, recon, mode, pd);
+  const long v = (long)cus * std::min(kLineBlocks, ql_blocks_per_cu<T>(n1, rot, recon, mode, pd));
   cache[key] = v;
   return v;
 }
@@ -788,9 +795,10 @@ static int ql_stage(const boltx_grid* g, const boltx_physics* ph, const boltx_st
   else if (st->a == 0.0 && st->b == 1.0) mode = w_is_u ? QL_WU_PLAIN : QL_W_PLAIN;
   const int pd = sp.source ? sp.p_dim : 0;
   const long groups = (sp.P + 3) / 4;
-  q.nseg = ql_segments(g->n_q2, groups, ql_slots<T>(g->n_q1, ph->recon_q, mode, pd));
+  const bool rot = ql_rot_applies<T>(q);
+  q.nseg = ql_segments(g->n_q2, groups, ql_slots<T>(g->n_q1, rot, ph->recon_q, mode, pd));
   const int nb = (int)(groups * q.nseg);
-  ql_launch<T>(q, ph->recon_q, nb, mode, pd, s);
+  ql_launch<T>(q, rot, ph->recon_q, nb, mode, pd, s);
   if ((rc = launch_status("qline_kernel"))) return rc;
   if (st->mom_out)
     return ql_moments<T>(g, sp, st->out, st->mom_out, part,

@@ -3,6 +3,6 @@
 #include "ql_launch.h"
 
 namespace bx {
-template void ql_launch<float>(const QLParams&, int, int, int, int, hipStream_t);
-template int ql_blocks_per_cu<float>(int, int, int, int);
+template void ql_launch<float>(const QLParams&, bool, int, int, int, int, hipStream_t);
+template int ql_blocks_per_cu<float>(int, bool, int, int, int);
 }

@@ -3,6 +3,6 @@
 #include "ql_launch.h"
 
 namespace bx {
-template void ql_launch<double>(const QLParams&, int, int, int, int, hipStream_t);
-template int ql_blocks_per_cu<double>(int, int, int, int);
+template void ql_launch<double>(const QLParams&, bool, int, int, int, int, hipStream_t);
+template int ql_blocks_per_cu<double>(int, bool, int, int, int);
 }

@@ -8,8 +8,8 @@
 //  * q2: a 6-row register window per cell (five stencil rows and the row
 //    loaded ahead); the WENO indicator and the upwind flux of each q2 face are
 //    computed once and carried to the next row;
-//  * q1: the row, its indicators and its face fluxes go through a
-//    wave-private LDS line (no workgroup barrier), so every q1 indicator and
+//  * q1: the row, its indicators and its face fluxes go through DPP rotates or
+//    a wave-private LDS line (no workgroup barrier), so every q1 indicator and
 //    face is computed once;
 //  * one p per wave makes the upwind direction of both axes a scalar branch,
 //    and every global access is a coalesced run along q1;
@@ -137,6 +137,51 @@ __device__ inline void ql_put(T* line, int i, bool live, int n1, T v) {
   if (i >= n1 - QL_HALO) line[i - n1] = v;
 }
 
+// A value held by the wave rotated by one lane, lane 63's neighbour being lane
+// 0: the periodic q1 neighbour where a line fills the wave.  UP: lane l gets
+// lane l+1's value, otherwise lane l-1's (DPP wave rotates).  All 64 lanes must
+// be active.
+template <bool UP, typename T>
+__device__ __forceinline__ T ql_rot(T v) {
+  constexpr int ctrl = UP ? 0x134 : 0x13c;  // wave_rol:1, wave_ror:1
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(
+        T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, true));
+  } else {
+    typedef int I2 __attribute__((ext_vector_type(2)));
+    I2 x = __builtin_bit_cast(I2, v);
+    x[0] = __builtin_amdgcn_update_dpp(0, x[0], ctrl, 0xf, 0xf, true);
+    x[1] = __builtin_amdgcn_update_dpp(0, x[1], ctrl, 0xf, 0xf, true);
+    return __builtin_bit_cast(T, x);
+  }
+}
+
+// x[LO + k] = the lane's own NR cells of a line (cell lane * NR + k); fills
+// the LO cells before and the HI cells after them from the neighbouring lanes.
+template <int NR, int LO, int HI, typename T>
+__device__ __forceinline__ void ql_neighbours(T (&x)[LO + NR + HI]) {
+#pragma unroll
+  for (int j = 0; j < HI; ++j) x[LO + NR + j] = ql_rot<true>(x[LO + j]);
+#pragma unroll
+  for (int j = LO - 1; j >= 0; --j) x[j] = ql_rot<false>(x[j + NR]);
+}
+
+// The lane's NR cells of a row: one vector load of adjacent cells (ROT), or
+// cells i1[k] = lane + 64 k.
+template <typename T, int NR, bool ROT, bool NT>
+__device__ __forceinline__ void ql_load(const T* row, const int (&i1)[NR], T (&v)[NR]) {
+  if constexpr (ROT) {
+    typedef T V __attribute__((ext_vector_type(NR)));
+    const V* a = (const V*)(row + i1[0]);
+    const V x = NT ? __builtin_nontemporal_load(a) : *a;
+#pragma unroll
+    for (int k = 0; k < NR; ++k) v[k] = x[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < NR; ++k) v[k] = NT ? __builtin_nontemporal_load(row + i1[k]) : row[i1[k]];
+  }
+}
+
 // Stage forms the march is specialised for (out = a*un + b*(w + cdt*L(u))):
 // QL_WU_PLAIN  w == u, a == 0, b == 1  (first stage of either stepper)
 // QL_WU_COMB   w == u, a != 0          (SSP-RK3 stages 2 and 3)
@@ -158,8 +203,14 @@ enum QlMode : int { QL_WU_PLAIN = 0, QL_WU_COMB = 1, QL_W_PLAIN = 2, QL_GENERAL 
 // the face uses the window's centre y2 and the indicators of y1, y2, y3, and
 // the flux through face r-1/2 is carried from the previous row.  Along q1 the
 // row goes through the wave's LDS line: values, then indicators, then the flux
-// through each cell's lower face.
-template <typename T, int R, int NR, bool P1, bool P2, int MODE, int PD>
+// through each cell's lower face.  With ROT (n1 = 64 NR exactly, pointers
+// aligned to a lane's cells) a lane holds NR adjacent cells and takes the
+// values, indicators and fluxes of its neighbours by DPP rotates instead:
+// 7 rotates for 2 cells where the LDS line takes 26 LDS operations and three
+// dependent round trips a row, which 4 waves per SIMD do not hide (FP64, 128^2 q
+// x 48^2 p: the first stage 197 -> 173 us, at 3.5 TB/s bound by FP64 issue; the
+// others 197 -> 185 us, 4.9 TB/s, the rate of a copy).
+template <typename T, int R, int NR, bool ROT, bool P1, bool P2, int MODE, int PD>
 __device__ __forceinline__ void ql_march(const QLParams& q, int p, int seg, int lane, T* fl, T* kl,
                                          T* sl) {
   const int n1 = q.n1, n2 = q.n2;
@@ -196,8 +247,8 @@ __device__ __forceinline__ void ql_march(const QLParams& q, int p, int seg, int 
   bool live[NR];
 #pragma unroll
   for (int k = 0; k < NR; ++k) {
-    i1[k] = lane + 64 * k;
-    live[k] = i1[k] < n1;
+    i1[k] = ROT ? lane * NR + k : lane + 64 * k;
+    live[k] = ROT || i1[k] < n1;
     if (!live[k]) i1[k] = 0;
   }
 
@@ -214,23 +265,21 @@ __device__ __forceinline__ void ql_march(const QLParams& q, int p, int seg, int 
     T z[NR];
     int rr = qm_mod(r0 + B - 1, n2);
     const T* row = u + rr * rowP;
-#pragma unroll
-    for (int k = 0; k < NR; ++k) z[k] = row[i1[k]];
+    ql_load<T, NR, ROT, false>(row, i1, z);
 #pragma unroll
     for (int j = 0; j < 5; ++j) {
       rr = rr + 1 == n2 ? 0 : rr + 1;
       row = u + rr * rowP;
-#pragma unroll
-      for (int k = 0; k < NR; ++k) Y[j][k] = row[i1[k]];
+      ql_load<T, NR, ROT, false>(row, i1, Y[j]);
     }
     const int rs0 = qm_mod(r0, n2);
+    if (!w_is_u) ql_load<T, NR, ROT, false>(wv + rs0 * rowP, i1, WC[0]);
+    if (use_un) ql_load<T, NR, ROT, false>(unv + rs0 * rowP, i1, UNC[0]);
+    if (src) ql_load<T, NR, ROT, false>(t1p + (long)rs0 * n1, i1, TC1[0]);
+    if (src2) ql_load<T, NR, ROT, false>(t2p + (long)rs0 * n1, i1, TC2[0]);
+    if (src3) ql_load<T, NR, ROT, false>(t3p + (long)rs0 * n1, i1, TC3[0]);
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
-      WC[0][k] = w_is_u ? T(0) : wv[rs0 * rowP + i1[k]];
-      UNC[0][k] = use_un ? unv[rs0 * rowP + i1[k]] : T(0);
-      TC1[0][k] = src ? t1p[(long)rs0 * n1 + i1[k]] : T(0);
-      TC2[0][k] = src2 ? t2p[(long)rs0 * n1 + i1[k]] : T(0);
-      TC3[0][k] = src3 ? t3p[(long)rs0 * n1 + i1[k]] : T(0);
       S2[0][k] = T(0);
       K[0][k] = K[1][k] = T(0);
       if (do_q2) {
@@ -273,15 +322,12 @@ __device__ __forceinline__ void ql_march(const QLParams& q, int p, int seg, int 
       const T* w1 = wv + rnx1 * rowP;
       const T* un1 = unv + rnx1 * rowP;
       const long tq = (long)rnx1 * n1;
-#pragma unroll
-      for (int k = 0; k < NR; ++k) {
-        Y[yl][k] = __builtin_nontemporal_load(uw + i1[k]);
-        WC[nx][k] = w_is_u ? T(0) : __builtin_nontemporal_load(w1 + i1[k]);
-        UNC[nx][k] = use_un ? __builtin_nontemporal_load(un1 + i1[k]) : T(0);
-        TC1[nx][k] = src ? t1p[tq + i1[k]] : T(0);
-        TC2[nx][k] = src2 ? t2p[tq + i1[k]] : T(0);
-        TC3[nx][k] = src3 ? t3p[tq + i1[k]] : T(0);
-      }
+      ql_load<T, NR, ROT, true>(uw, i1, Y[yl]);
+      if (!w_is_u) ql_load<T, NR, ROT, true>(w1, i1, WC[nx]);
+      if (use_un) ql_load<T, NR, ROT, true>(un1, i1, UNC[nx]);
+      if (src) ql_load<T, NR, ROT, false>(t1p + tq, i1, TC1[nx]);
+      if (src2) ql_load<T, NR, ROT, false>(t2p + tq, i1, TC2[nx]);
+      if (src3) ql_load<T, NR, ROT, false>(t3p + tq, i1, TC3[nx]);
     }
     T d[NR], fc[NR];
 #pragma unroll
@@ -299,7 +345,33 @@ __device__ __forceinline__ void ql_march(const QLParams& q, int p, int seg, int 
         S2[nx][k] = f2p;
       }
     }
-    if (do_q1) {
+    if constexpr (ROT) {
+      // as below, with x[LO + k], kx[LO + k] the lane's own cells
+      constexpr int LO = P1 ? 3 : 2, HI = P1 ? 1 : 2;
+      T x[LO + NR + HI];
+#pragma unroll
+      for (int k = 0; k < NR; ++k) x[LO + k] = fc[k];
+      ql_neighbours<NR, LO, HI>(x);
+      constexpr int KLO = P1 ? 2 : 1, KHI = P1 ? 0 : 1;
+      T kx[KLO + NR + KHI], sx[NR + 1];
+#pragma unroll
+      for (int k = 0; k < NR; ++k)
+        kx[KLO + k] = ql_kappa<R, T>(x[LO + k - 1], x[LO + k], x[LO + k + 1]);
+      if constexpr (R == RC_WENO5) {
+        ql_neighbours<NR, KLO, KHI>(kx);
+      } else {
+#pragma unroll
+        for (int k = 0; k < KLO; ++k) kx[k] = T(0);
+        if constexpr (KHI == 1) kx[KLO + NR] = T(0);
+      }
+#pragma unroll
+      for (int k = 0; k < NR; ++k)
+        sx[k] = ql_flux(C1, ql_face<R, P1, T>(x[k], x[k + 1], x[k + 2], x[k + 3], x[k + 4], kx[k],
+                                              kx[k + 1], kx[k + 2]));
+      ql_neighbours<NR, 0, 1>(sx);
+#pragma unroll
+      for (int k = 0; k < NR; ++k) d[k] = ql_fma(sx[k] - sx[k + 1], tinv1, -d[k]);
+    } else if (do_q1) {
 #pragma unroll
       for (int k = 0; k < NR; ++k) {
         fl[a1[k]] = fc[k];
@@ -360,6 +432,7 @@ __device__ __forceinline__ void ql_march(const QLParams& q, int p, int seg, int 
     }
     // source, RK combination, store
     T* orow = outv + rcur * rowP;
+    T xo[NR];
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
       const T f = fc[k];
@@ -371,8 +444,19 @@ __device__ __forceinline__ void ql_march(const QLParams& q, int p, int seg, int 
         dk = ql_fma(fmb - f, tinvtau, dk);
       }
       const T tv = ql_fma(dk, tcdt, w_is_u ? f : WC[cu][k]);
-      const T x = use_un ? ql_fma(ta, UNC[cu][k], tb * tv) : (plain ? tv : tb * tv);
-      if (live[k]) orow[i1[k]] = x;  // kept in the caches for the moment pass
+      xo[k] = use_un ? ql_fma(ta, UNC[cu][k], tb * tv) : (plain ? tv : tb * tv);
+    }
+    // (kept in the caches for the moment pass)
+    if constexpr (ROT) {
+      typedef T V __attribute__((ext_vector_type(NR)));
+      V v;
+#pragma unroll
+      for (int k = 0; k < NR; ++k) v[k] = xo[k];
+      *(V*)(orow + i1[0]) = v;
+    } else {
+#pragma unroll
+      for (int k = 0; k < NR; ++k)
+        if (live[k]) orow[i1[k]] = xo[k];
     }
     rcur = rnx1;
     rnx1 = rnx1 + 1 == n2 ? 0 : rnx1 + 1;
@@ -400,13 +484,16 @@ __device__ __forceinline__ void ql_march(const QLParams& q, int p, int seg, int 
 // next segment) and spread over the eight XCDs in contiguous ranges, so the
 // p-cells running together on one XCD share a segment and its rows of the
 // Maxwellian tables stay in that XCD's L2.
-template <typename T, int R, int NR, int MODE, int PD>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void qline_kernel(QLParams q) {
+// Waves per SIMD: 4, or 2 where a lane holds 4 FP64 cells (204 VGPRs; at 4 waves
+// it spills 420 bytes a lane: 3152 -> 1090 us per step at 256 x 128 q, 40^2 p).
+template <typename T, int R, int NR, bool ROT, int MODE, int PD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NR * sizeof(T) > 16 ? 2 : 4))) void qline_kernel(QLParams q) {
+  constexpr int kLine = ROT ? QL_HALO + 1 : NR * 64 + 2 * QL_HALO + 64;
   // wave-private q1 lines with three halo cells on each side: row values,
   // q1 indicator quantities and lower-face states
-  __shared__ T fl[4][NR * 64 + 2 * QL_HALO + 64];
-  __shared__ T kl[4][NR * 64 + 2 * QL_HALO + 64];
-  __shared__ T sl[4][NR * 64 + 2 * QL_HALO + 64];
+  __shared__ T fl[4][kLine];
+  __shared__ T kl[4][kLine];
+  __shared__ T sl[4][kLine];
   // the wave index is uniform across the wave: keep it (and all that derives
   // from it: p-cell, velocities, row pointers) in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -423,11 +510,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void q
   T* k = kl[wave] + QL_HALO;
   T* s = sl[wave] + QL_HALO;
   if (pos1) {
-    if (pos2) ql_march<T, R, NR, true, true, MODE, PD>(q, p, seg, lane, f, k, s);
-    else ql_march<T, R, NR, true, false, MODE, PD>(q, p, seg, lane, f, k, s);
+    if (pos2) ql_march<T, R, NR, ROT, true, true, MODE, PD>(q, p, seg, lane, f, k, s);
+    else ql_march<T, R, NR, ROT, true, false, MODE, PD>(q, p, seg, lane, f, k, s);
   } else {
-    if (pos2) ql_march<T, R, NR, false, true, MODE, PD>(q, p, seg, lane, f, k, s);
-    else ql_march<T, R, NR, false, false, MODE, PD>(q, p, seg, lane, f, k, s);
+    if (pos2) ql_march<T, R, NR, ROT, false, true, MODE, PD>(q, p, seg, lane, f, k, s);
+    else ql_march<T, R, NR, ROT, false, false, MODE, PD>(q, p, seg, lane, f, k, s);
   }
 }
 

@@ -257,7 +257,7 @@ def run_em(steps=10, warmup=2):
     SSP-RK3 dt = 2e-4 with the fields advanced once per step (Yee FDTD);
     FP32-bulk and plain FP64, with the FP32-bulk error against the FP64 run
     after the same steps.  The roofline is that of the stage kernel
-    (qcell_kernel with p-advection) at the algorithmic bytes of an SSP-RK3
+    (qdiff_kernel and pplane_kernel together) at the algorithmic bytes of an SSP-RK3
     stage (8/3 f-passes), beside the whole step's algorithmic rate."""
     import torch
     from tests.cases import case_2d3v, hip_solver
@@ -277,15 +277,18 @@ def run_em(steps=10, warmup=2):
         achieved = 8 / 3 * cells * esz / stage_s / 1e9
         ms_step = _median(ms)
         step_gbs = 8 * esz * cells / (ms_step / 1e3) / 1e9
+        seq = _traffic("em_" + prec, "bytes_per_sequence")
+        per_stage = seq / 3 if seq else None
         out[prec] = {"ms_per_step": ms_step, "ms_per_step_repeats": ms,
                      "warmup_steps_run": warm, "value": cells / (ms_step / 1e3),
                      "stage_launch_ms_avg": stage_s * 1e3,
                      "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                                   "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-                                  "traffic": _traffic("em_" + prec),
+                                  "traffic": per_stage,
                                   "step_achieved": step_gbs,
                                   "step_frac": step_gbs / HBM_PEAK_GBS},
-                     "kernel": "qcell_kernel (stage with p-advection, 8/3 f-passes per launch)"}
+                     "kernel": "qdiff_kernel + pplane_kernel (stage with p-advection, 8/3 "
+                               "f-passes per stage)"}
         del s
     n_err = 20
     return {"workload": "2D3V EM 64^2 q x 24^3 p, PPM q / WENO5 p, LLF, BGK tau=0.1, "
@@ -457,7 +460,7 @@ def probe(which):
     read and written: the counter calibration), then one SSP-RK3 step of the
     headline workload (``fp64``, ``fp32-bulk``: three qline_kernel stages
     and their moment passes) or of the 2D3V electromagnetic one (``em-fp64``,
-    ``em-fp32-bulk``: three qcell_kernel stages)."""
+    ``em-fp32-bulk``: three stages of a qdiff_kernel and a pplane_kernel)."""
     import torch
     from tests.cases import case_2d2v, case_2d3v, case_c5, hip_solver
     x = torch.ones(32 * 1024 * 1024, dtype=torch.float64, device="cuda")  # 256 MiB
@@ -488,7 +491,8 @@ def probe(which):
 
 def probe_algorithmic(which):
     """Algorithmic bytes of the probe's three stage launches: stage 1 reads
-    u and writes out, stages 2 and 3 also read un.  The ensemble's step
+    u and writes out, stages 2 and 3 also read un (with p-advection a stage is
+    two launches, the second carries its bytes).  The ensemble's step
     alternates stage and finalize launches; the finalize has no algorithmic
     bytes of its own (its traffic is the moment partials and tables)."""
     if which == "ensemble":
@@ -497,6 +501,8 @@ def probe_algorithmic(which):
         return [8 * cells, 0, 12 * cells, 0, 12 * cells, 0]
     cells = 64 * 64 * 24 ** 3 if which.startswith("em-") else 128 * 128 * 48 * 48
     esz = 4 if which.endswith("fp32-bulk") else 8
+    if which.startswith("em-"):
+        return [0, 2 * cells * esz, 0, 3 * cells * esz, 0, 3 * cells * esz]
     return [2 * cells * esz, 3 * cells * esz, 3 * cells * esz]
 
 
@@ -531,7 +537,7 @@ def main():
                                  extra={"tuning": list(ENSEMBLE_PROBE_TUNING)})
             print(json.dumps({w: e}, indent=1), flush=True)
             return
-        kernel = "qcell_kernel|qsweep_kernel" if w.startswith("em-") else "qline_kernel"
+        kernel = "qdiff_kernel|pplane_kernel" if w.startswith("em-") else "qline_kernel"
         key = "em_" + w[3:] if w.startswith("em-") else w
         e = traffic_from_pmc(key, args.traffic[0], args.traffic[1], kernel, probe_algorithmic(w))
         print(json.dumps({key: e}, indent=1), flush=True)

@@ -1303,6 +1303,12 @@ extern "C" int boltx_advance(int n, const boltx_state* sp, int stepper, double d
       const boltx_stage st = plan(i, k);
       if ((rc = check_stage(sp[i].grid, sp[i].phys, &st))) return rc;
     }
+    if (sp[i].grid->layout == BOLTX_LAYOUT_Q1_LINES) {
+      if (fields) return fail(BOLTX_EUNSUPPORTED, "p-advection needs the reference layout");
+      if (!sp[i].workspace) return fail(BOLTX_EINVAL, "the q1-line layout needs the workspace");
+      if (sp[i].grid->n_q1 > 1 && sp[i].grid->n_q1 < QL_HALO)
+        return fail(BOLTX_EUNSUPPORTED, "the q1-line layout needs n_q1 = 1 or n_q1 >= %d", QL_HALO);
+    }
     if (ghost_rows(sp[i].grid) > 0)
       for (int k = 0; k < 4; ++k)
         if (sp[i].grid->bc[k] == BOLTX_BC_DIRICHLET || sp[i].grid->bc[k] == BOLTX_BC_MIRROR_DIRICHLET)

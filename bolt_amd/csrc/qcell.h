@@ -11,6 +11,9 @@
 // the same function for this linear flux (C does not depend on f), so LLF
 // evaluates through the upwind state as well.
 //
+// Large problems of the reference layout take the marching stages instead
+// (psplit.h; the sizes are kSplitCells and kMarchCells in boltx.hip).
+//
 // Reference: df_dt_fvm.py:56-97 (q fluxes + source), 251-323 (p fluxes),
 // riemann.py:46-49, weno5.py:57-98, collision_operator.py:52-65.
 #pragma once

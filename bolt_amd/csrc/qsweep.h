@@ -28,6 +28,9 @@
 // pitch for n_p1 = 24, so a wave's 64 lines hit 64 distinct banks), the
 // accumulator in the same padded layout, and the Maxwellian factor tables.
 //
+// Serves problems below the size of the two-kernel stage (psplit.h, kSplitCells)
+// and p-blocks that it does not take.
+//
 // Reference: df_dt_fvm.py:251-323 (p fluxes), weno5.py:57-98,
 // riemann.py:46-49; the rest as qcell_kernel.
 #pragma once

@@ -132,8 +132,9 @@ int boltx_fvm_stage(const boltx_grid *grid, const boltx_physics *phys,
  * device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  stage->workspace must be NULL; the workspace lives
  * in a static device array of BOLTX_SCRATCH_BYTES that the library holds on
- * every GPU it runs on until the process ends.  A problem whose
- * boltx_workspace_size() exceeds it is rejected with BOLTX_EUNSUPPORTED.
+ * every GPU it runs on until the process ends (a stage whose workspace holds
+ * the q-part of L takes it there in smaller pieces).  A problem that needs more
+ * is rejected with BOLTX_EUNSUPPORTED.
  * Every call on one GPU shares that GPU's array: calls whose device work
  * overlaps (other streams, other host threads) race, so order them on one
  * stream.  Outputs equal those of boltx_fvm_stage bit for bit. */
@@ -206,9 +207,10 @@ int boltx_fill_ghosts(const boltx_grid *grid, const boltx_physics *phys, void *f
 
 /* Bytes of device workspace boltx_fvm_stage and boltx_moments use for this
  * problem (required in the q1-line layout, optional in the reference layout,
- * where it holds the sign-grouped p order and, with p-advection in three p
- * axes, the q-part of L between the stage's two kernels: up to one more
- * f-sized array, at most 2 GiB), and its one-time set-up.  The
+ * where it holds the sign-grouped p order and, for large problems, with
+ * p-advection in three p axes the q-part of L between the stage's two kernels
+ * (up to one more f-sized array, at most 2 GiB), without p-advection the
+ * Maxwellian tables and moment partials), and its one-time set-up.  The
  * reference has no counterpart: ArrayFire allocates its temporaries itself;
  * here the caller owns all device memory. */
 size_t boltx_workspace_size(const boltx_grid *grid, const boltx_physics *phys);

@@ -549,8 +549,12 @@ static size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 // p-cells to fill its waves and enough cells that its three launches per stage
 // beat the one of the slab kernel.  FP32 WENO5 stays with the slab kernel, whose
 // rounding of the weights its results have always had.
-static bool qmarch_applies(const boltx_physics* ph, size_t P, double cells) {
+// FP32 with ghost rows takes it from 4 kMarchCells (mirror walls, PPM: 60 x 67 q,
+// 33 x 26 p 192 us in the slab kernel / 204 in the march, 96 x 60 q, 30^2 p
+// 229 / 230, 90^2 q, 36^2 p 433 / 351).
+static bool qmarch_applies(const boltx_physics* ph, size_t P, double cells, bool ghosts) {
   if (ph->precision != BOLTX_FP64 && ph->recon_q == RC_WENO5) return false;
+  if (ph->precision != BOLTX_FP64 && ghosts && cells < 4 * kMarchCells) return false;
   const bool light = ph->recon_q == RC_PC || ph->recon_q == RC_MINMOD;
   return P >= 48 && cells >= (light ? kMarchCellsMinmod : kMarchCells);
 }
@@ -577,7 +581,7 @@ static RefWorkspace ref_workspace(const boltx_grid* g, const boltx_physics* ph, 
     row = P * g->n_q1 * esz;
     prow = slabs * 3 * sizeof(double) * g->n_q1;
   } else {
-    if (!qmarch_applies(ph, P, cells)) return w;
+    if (!qmarch_applies(ph, P, cells, ghost_rows(g) > 0)) return w;
     row = (size_t)(g->n_p1 + g->n_p2 + g->n_p3) * g->n_q1 * esz;
     prow = slabs * 5 * sizeof(double) * g->n_q1;
     if (P * g->n_q1 * esz > kSplitChunkScratch) return w;  // 32-bit offsets in a row of q-cells

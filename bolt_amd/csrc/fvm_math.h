@@ -16,6 +16,11 @@
 
 namespace bx {
 
+// An explicit fused multiply-add, where the rounding must not depend on what the
+// compiler contracts.
+__host__ __device__ inline double ql_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__host__ __device__ inline float ql_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
 enum Recon : int { RC_PC = 0, RC_MINMOD = 1, RC_PPM = 2, RC_WENO5 = 3 };
 enum Riemann : int { RS_UPWIND = 0, RS_LLF = 1 };
 

@@ -158,6 +158,7 @@ __device__ inline void qc_finish(const StageParams& sp, int q, double (&acc)[5],
   for (int k = 0; k < 3; ++k) v[5 + k] = jac[k];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
+    if (k >= 5 && !cur) break;
     double x = v[k];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
@@ -184,25 +185,29 @@ __global__ __launch_bounds__(NT) void qcell_kernel(QCParams qp) {
   constexpr int NW = NT / 64;
   extern __shared__ unsigned char smem[];
   __shared__ double red[8][NW];
+  __shared__ double pref;
   const StageParams& sp = qp.sp;
   T* tab = reinterpret_cast<T*>(smem);
   T* blk = tab + (sp.n_p1 + sp.n_p2 + sp.n_p3);
   const int q = qc_order(sp, blockIdx.x, gridDim.x);
   QCell<T> c;
   qcell_neighbours(sp, q, c);
-  c.pref = 0.0;
   c.e1 = c.e2 = c.e3 = tab;
   if (sp.source) {
+    // the prefactor (a pow) by wave 0, the factors starting at waves 1, 2, 3: the
+    // long FP64 chains run side by side instead of one after another (with the
+    // loads of the loop below issued together, a step at 48 x 40 q, 20 x 24 p,
+    // FP64 WENO5 with walls: 110.6 -> 105.3 us)
     const BgkCell b = qcell_bgk(sp, q);
-    c.pref = maxwell_prefactor(b, sp.mass, sp.kB, sp.p_dim);
+    if (threadIdx.x == 0) pref = maxwell_prefactor(b, sp.mass, sp.kB, sp.p_dim);
     T* e1 = tab;
     T* e2 = tab + sp.n_p1;
     T* e3 = e2 + sp.n_p2;
-    for (int i = threadIdx.x; i < sp.n_p1; i += blockDim.x)
+    for (int i = (threadIdx.x + NT - 64) % NT; i < sp.n_p1; i += NT)
       e1[i] = T(maxwell_factor(centre(sp.p1s, i, sp.dp1), b.u1, b.T, sp.mass, sp.kB));
-    for (int i = threadIdx.x; i < sp.n_p2; i += blockDim.x)
+    for (int i = (threadIdx.x + NT - 128) % NT; i < sp.n_p2; i += NT)
       e2[i] = T(maxwell_factor(centre(sp.p2s, i, sp.dp2), b.u2, b.T, sp.mass, sp.kB));
-    for (int i = threadIdx.x; i < sp.n_p3; i += blockDim.x)
+    for (int i = (threadIdx.x + NT - 192) % NT; i < sp.n_p3; i += NT)
       e3[i] = T(maxwell_factor(centre(sp.p3s, i, sp.dp3), b.u3, b.T, sp.mass, sp.kB));
     c.e1 = e1;
     c.e2 = e2;
@@ -215,6 +220,7 @@ __global__ __launch_bounds__(NT) void qcell_kernel(QCParams qp) {
     for (int p = threadIdx.x; p < sp.P; p += blockDim.x) blk[p] = u[(long)q * P + p];
   }
   __syncthreads();
+  c.pref = sp.source ? pref : 0.0;
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const T* wv = (const T*)sp.w;
@@ -245,7 +251,10 @@ __global__ __launch_bounds__(NT) void qcell_kernel(QCParams qp) {
     const double v3 = centre(sp.p3s, j3, sp.dp3);
     const bool pos1 = __builtin_amdgcn_readfirstlane(int(v1 > 0.0)) != 0;
     const bool pos2 = __builtin_amdgcn_readfirstlane(int(v2 > 0.0)) != 0;
+    // every load before the stencils, so none waits behind them
     const T f = u[base + p];
+    const T wval = w_is_u ? f : wv[base + p];
+    const T unval = use_un ? unv[base + p] : T(0);
     T t1 = T(0), t2 = T(0), s1 = f, s2 = f;
     if (sp.n_q1 > 1) {
       T a[7];
@@ -289,9 +298,8 @@ __global__ __launch_bounds__(NT) void qcell_kernel(QCParams qp) {
       }
       d = d - dp;
     }
-    const T wval = w_is_u ? f : wv[base + p];
     const T tv = wval + d * tcdt;
-    const T x = use_un ? ta * unv[base + p] + tb * tv : (sp.b == 1.0 ? tv : tb * tv);
+    const T x = use_un ? ql_fma(tb, tv, ta * unval) : (sp.b == 1.0 ? tv : tb * tv);
     if (valid) {
       outv[base + p] = x;
       const double xd = double(x);

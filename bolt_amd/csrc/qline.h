@@ -48,9 +48,7 @@ struct QLParams {
 // (one per register rotation), and the compiler's choice of which product of
 // a*b + c*d to fuse depends on how often each product is reused, which
 // differs between copies; so the march's functions evaluate with contraction
-// off and fuse explicitly, and every row rounds the same way in every copy.
-__host__ __device__ inline double ql_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
-__host__ __device__ inline float ql_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+// off and fuse explicitly (ql_fma), and every row rounds the same way in every copy.
 
 template <int R, typename T>
 __host__ __device__ inline T ql_kappa(T a, T b, T c) {

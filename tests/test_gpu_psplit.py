@@ -137,7 +137,7 @@ def _fields_off(nq, np_, recon, precision, walls=""):
     ((2051, 1), (32, 65, 1), "piecewise-constant", "general", ""),
     ((33, 34), (12, 11, 13), "ppm", "general", ""),
     ((50, 47), (27, 27, 1), "weno5", "combine", "1"),
-    ((47, 50), (27, 27, 1), "ppm", "first", "2"),
+    ((93, 95), (27, 27, 1), "ppm", "first", "2"),
     ((45, 51), (30, 26, 1), "weno5", "midpoint", "12"),
 ])
 @pytest.mark.parametrize("precision", ["fp64", "fp32-bulk"])
